@@ -84,7 +84,8 @@ def sum_by_structure(soff: torch.Tensor, x: torch.Tensor, out: torch.Tensor | No
     """Per-structure sums [n_struct, width] of x's rows, atoms soff[b] .. soff[b+1]-1."""
     lib = _lib.load()
     NS, W = int(soff.numel()) - 1, int(x.shape[1])
-    out = torch.zeros((NS, W), dtype=torch.float64, device=x.device) if out is None else out
+    if out is None:  # every element is written unless they are added onto
+        out = (torch.zeros if accumulate else torch.empty)((NS, W), dtype=torch.float64, device=x.device)
     _lib.check(lib.pet_sum_by_structure(NS, W, soff.data_ptr(), _f64(x, "x", x.numel()), _f64(out, "out", NS * W),
                                         int(accumulate), _stream()), "pet_sum_by_structure")
     return out

@@ -145,6 +145,39 @@ def test_edge_grad_dead_rows_and_neighbour_only_atoms(device):
     assert np.all(forces.cpu().numpy()[N:] == 0.0) and np.all(vir.cpu().numpy()[N:] == 0.0)
 
 
+@pytest.mark.parametrize("counts", [[0, 1, 63, 0], [64, 65, 127], [128, 129, 2, 300]])
+def test_fold_chunks_of_edges(device, counts):
+    """Atoms with no edge, and edge counts around the 64 a wavefront takes at
+    once; some edges without a reverse. fp64 sums in the oracle's order: what
+    may differ is a multiply-add's rounding, 1e-12 of the largest sum."""
+    print(f"[gpu] fold chunks {counts}", flush=True)
+    rng = np.random.default_rng(11)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    N, E = len(counts), int(off[-1])
+    vec, g = rng.standard_normal((E, 3)), rng.standard_normal((E, 3))
+    rev = rng.integers(-1, E, E).astype(np.int32)
+    center = np.repeat(np.arange(N), counts).astype(np.int32)
+    one = np.ones(E)
+    host = systems.PackedEdges(off, center, center, rev, vec, one, one, one.astype(np.float32))
+    dpk = F.PackedEdges.from_host(host, device)
+    forces, vir = F.fold_edge_gradients(dpk, N, dev(g, device), scale=0.5)
+    torch.cuda.synchronize()
+    rf, rv = oracle.fold(N, off, rev, vec, g, scale=0.5)
+    assert rel(forces.cpu().numpy(), rf) <= 1e-12
+    assert rel(vir.cpu().numpy(), rv) <= 1e-12
+
+
+@pytest.mark.parametrize("size", [1, 63, 65, 511, 512, 513, 1728])
+def test_sum_by_structure_sizes(device, size):
+    """One structure around the 8 x 64 atoms a wavefront's lanes load at once."""
+    print(f"[gpu] sum_by_structure {size}", flush=True)
+    x = np.random.default_rng(size).standard_normal((size + 5, 9))
+    soff = np.array([2, 2 + size, 5 + size], dtype=np.int32)
+    out = F.sum_by_structure(dev(soff, device), dev(x, device))
+    torch.cuda.synchronize()
+    assert rel(out.cpu().numpy(), oracle.struct_sum(soff, x)) <= 1e-12
+
+
 def test_sum_by_structure(device):
     print("[gpu] sum_by_structure", flush=True)
     rng = np.random.default_rng(3)
