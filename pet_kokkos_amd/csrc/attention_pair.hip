@@ -18,8 +18,8 @@
 //   holding key 16w + c against queries 16I + 4g + r (lane l = (c, g) =
 //   (l % 16, l / 16), register r of the result);
 //   P and dS, scaled and split in registers, are then already the b operand
-//   of the 16x16x16 instruction for dV_w^T += dO_I^T P and dK_w^T += Q_I^T dS
-//   (k = the block's 16 queries), so the key block's dK and dV never leave the
+//   for dV_w^T += dO_I^T P and dK_w^T += Q_I^T dS (k = the block's 16 queries,
+//   mfma_block), so the key block's dK and dV never leave the
 //   wave's registers; only dS goes through LDS to the owner of query block
 //   I, which adds dQ_I^T += K_w^T dS^T after the step's barrier.
 // Every product is formed once, every output has one owner summing in a fixed
@@ -69,19 +69,29 @@ using pet_split::u4;
 
 namespace {
 
-constexpr int kPairHD = 32;
-constexpr int kPairMaxWaves = 8;  // 128 slots; beyond, the tile-exchange kernel
+// Waves a workgroup (16 slots each): every count up to 9, then the next even
+// one (pair_waves), up to 256 slots -- or as far as the planes fit the LDS (the
+// backward at head_dim 64: 160 slots). Past 128 slots a CU holds one backward
+// workgroup (two at nine waves), still well ahead of the fp32 tile-exchange
+// kernel, whose products take eight instructions where the pairs take three:
+// 640 atoms of 180 neighbours on MI355X (14 waves, d 256), backward 720 -> 490
+// us (427 with mfma_block), forward 207 -> 173; S 143 (nine waves) 373 -> 280
+// and 114 -> 100.
+constexpr int kPairMaxWaves = 16;
+constexpr int pair_waves(int NW) { return NW <= 9 ? NW : (NW + 1) & ~1; }
 
 struct PairLds {
   static constexpr int TP = 20;  // halves a dS tile row (16 queries, 4 of pad)
   static constexpr int TS = 16 * TP;  // halves a tile part
   // The planes token-major (a token's dims a row, tok_off: a lane's 8 dims
-  // one 16-byte store), rows padded at head_dim 32
-  static constexpr bool pad(int HD) { return HD <= 32; }
+  // one 16-byte store), rows padded at head_dim 32 -- but not with nine waves
+  // (unpadded, 80,352 bytes, a second workgroup fits the CU) nor with sixteen
+  // (padded rows pass the 160 KB)
+  static constexpr bool pad(int HD, int NW) { return HD <= 32 && NW != 9 && NW != 16; }
   int R, PT;  // rows; plane pitch in halves
   size_t pl, st, red, tb, bytes;
   __host__ __device__ constexpr PairLds(int HD, int NW)
-      : R(16 * NW), PT(pad(HD) ? HD + 8 : HD), pl(0),
+      : R(16 * NW), PT(pad(HD, NW) ? HD + 8 : HD), pl(0),
         st(pl + size_t(6) * 16 * NW * PT * 2),  // 6 planes: Q, dO, K, each hi then lo
         red(st + size_t(3) * R * 4),            // 8 words a wave: its maxima
         tb(red + size_t(8) * NW * 4), bytes(tb + size_t(2) * NW * 2 * TS * 2) {}
@@ -212,6 +222,28 @@ __device__ __forceinline__ void qkv_get8(const float* qkv, int64_t ldq, size_t r
 }
 }  // namespace
 
+// c += a.b over one 16-row block from fp16 pairs on the 16x16x32 instruction,
+// which takes the time of a 16x16x16 one (17 against 18 cycles a SIMD measured
+// on MI355X): the lower four k-slots of a lane carry a's lo parts, the upper
+// four its hi parts, so that with b1 = (b_hi, b_lo) one instruction is a_lo
+// b_hi + a_hi b_lo and with b2 = (0, b_hi) the next a_hi b_hi -- two
+// instructions where the 16x16x16 form (LOHI false) takes three. Its operand
+// quads take registers and copies the backward at head_dim 32 and up to eight
+// waves does not have to spare (held to 80 registers it spilled 12 bytes:
+// 1728 atoms of 70 neighbours 242 -> 250 us); past eight waves, where the
+// matrix work a wave grows with the atom, and at head_dim 64 it pays (640
+// atoms of 180 neighbours, d 256, backward 490 -> 427 us; 1000 of 70, 8 heads
+// of 64, 339 -> 330).
+template <bool LOHI>
+__device__ __forceinline__ f4 mfma_block(const u2& ah, const u2& al, const u2& bh, const u2& bl, f4 c) {
+  if constexpr (!LOHI) {
+    return mfma3_16(ah, al, bh, bl, c);
+  } else {
+    const u4 a = {al[0], al[1], ah[0], ah[1]}, b1 = {bh[0], bh[1], bl[0], bl[1]}, b2 = {0u, 0u, bh[0], bh[1]};
+    return pet_split::mfma_h(a, b2, pet_split::mfma_h(a, b1, c));
+  }
+}
+
 // The backward's arguments (one launch).
 struct PairBwdArgs {
   const float* qkv;
@@ -304,7 +336,7 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
   constexpr int PT = L.PT, TP = PairLds::TP, TS = PairLds::TS;
   _Float16* planes = reinterpret_cast<_Float16*>(lds + L.pl);
   constexpr int PS = L.R * PT;  // halves a plane part
-  constexpr bool PAD = PairLds::pad(HD);
+  constexpr bool PAD = PairLds::pad(HD, NW), LOHI = HD > 32 || NW > 8;  // mfma_block
   _Float16* QTh = planes;
   _Float16* GTh = planes + 2 * PS;
   _Float16* KTh = planes + 4 * PS;
@@ -451,8 +483,8 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
       const int o = tok_off<HD, PAD>(16 * I + 4 * g + (c >> 2), 2 * t + ((c & 3) >> 1)) + 4 * (c & 1);
       const u2 gth = lds_tr16(GTh + o), gtl = lds_tr16(GTh + PS + o), qth = lds_tr16(QTh + o),
                qtl = lds_tr16(QTh + PS + o);
-      dv[t] = mfma3_16(gth, gtl, ph, pl, dv[t]);
-      dk[t] = mfma3_16(qth, qtl, sh, sl, dk[t]);
+      dv[t] = mfma_block<LOHI>(gth, gtl, ph, pl, dv[t]);
+      dk[t] = mfma_block<LOHI>(qth, qtl, sh, sl, dk[t]);
     }
     // dS to query block I's owner: hi and lo tiles T[key c][query 4g + r],
     // read back transposed
@@ -474,7 +506,7 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
       // dim 16t + c of keys 16J + 4g .. + 3, read transposed
       const int o = tok_off<HD, PAD>(16 * J + 4 * g + (c >> 2), 2 * t + ((c & 3) >> 1)) + 4 * (c & 1);
       const u2 kth = lds_tr16(KTh + o), ktl = lds_tr16(KTh + PS + o);
-      dq[t] = mfma3_16(kth, ktl, bh, bl, dq[t]);
+      dq[t] = mfma_block<LOHI>(kth, ktl, bh, bl, dq[t]);
     }
   };
   // Software-pipelined: between two barriers a wave has phase 2 of the last
@@ -553,7 +585,8 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
 
 // One workgroup per item. BP: block pairs in place of qkv_adj (a.qpairs).
 template <int HD, int NW, bool XF, bool BP = false>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD > 32 ? 4 : NW >= 4 ? 6 : 5)))
+__global__ void __launch_bounds__(64 * NW)
+    __attribute__((amdgpu_waves_per_eu(HD > 32 || NW > 9 ? 4 : NW < 4 || NW == 9 ? 5 : 6)))
 attn_bwd_pair_kernel(PairBwdArgs a) {
   extern __shared__ float lds_f[];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
@@ -829,7 +862,7 @@ attn_fwd_pair_kernel(const float* __restrict__ qkv, int64_t ldq, const int* __re
 
 // ---- host side ---------------------------------------------------------------
 
-size_t pair_bwd_bytes(int HD, int NW) { return NW <= kPairMaxWaves ? PairLds(HD, NW).bytes : ~size_t(0); }
+size_t pair_bwd_bytes(int HD, int NW) { return NW <= kPairMaxWaves ? PairLds(HD, pair_waves(NW)).bytes : ~size_t(0); }
 
 const void* pair_bwd_kernel_ptr(int HD) {
   return HD == 64 ? reinterpret_cast<const void*>(attn_bwd_pair_kernel<64, 5, false>)
@@ -842,6 +875,7 @@ const void* pair_kernel(bool x) {
   return x ? reinterpret_cast<const void*>(attn_bwd_pair_kernel<HD, NW, true, BP>)
            : reinterpret_cast<const void*>(attn_bwd_pair_kernel<HD, NW, false, BP>);
 }
+// NW = pair_waves(waves); null where the planes do not fit (head_dim 64 past 10 waves)
 template <int HD, bool BP = false>
 const void* pair_kernel_nw(int NW, bool x) {
   switch (NW) {
@@ -852,8 +886,18 @@ const void* pair_kernel_nw(int NW, bool x) {
     case 5: return pair_kernel<HD, 5, BP>(x);
     case 6: return pair_kernel<HD, 6, BP>(x);
     case 7: return pair_kernel<HD, 7, BP>(x);
-    default: return pair_kernel<HD, 8, BP>(x);
+    case 8: return pair_kernel<HD, 8, BP>(x);
+    case 9: return pair_kernel<HD, 9, BP>(x);
+    case 10: return pair_kernel<HD, 10, BP>(x);
   }
+  if constexpr (HD <= 32) {
+    switch (NW) {
+      case 12: return pair_kernel<HD, 12, BP>(x);
+      case 14: return pair_kernel<HD, 14, BP>(x);
+      case 16: return pair_kernel<HD, 16, BP>(x);
+    }
+  }
+  return nullptr;
 }
 
 // The dynamic LDS limit of kernel k raised, once per device, to the largest
@@ -879,7 +923,7 @@ int pair_bwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
              const float* dmerged, int64_t ldg, const float* merged, int64_t ldm, const float* ml,
              const float* cf_seq, int64_t ldc, float* qkv_adj, int64_t lda, float* cfh, QkvXf xf, hipStream_t st,
              void* qpairs, int64_t prows) {
-  const int NW = (sh.slots + 15) / 16, HD = sh.head_dim;
+  const int NW = pair_waves((sh.slots + 15) / 16), HD = sh.head_dim;
   if (NW > kPairMaxWaves || (HD != 32 && HD != 64)) return PET_ATTN_ESLOTS;
   const int64_t items = int64_t(n1 - n0) * sh.heads;
   if (items == 0) return PET_ATTN_OK;
@@ -888,6 +932,7 @@ int pair_bwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
   const bool x = xf.rs || xf.b;
   const void* k = qpairs ? (HD == 64 ? pair_kernel_nw<64, true>(NW, x) : pair_kernel_nw<32, true>(NW, x))
                          : (HD == 64 ? pair_kernel_nw<64>(NW, x) : pair_kernel_nw<32>(NW, x));
+  if (!k) return PET_ATTN_ESLOTS;
   if (const int e = allow_lds_pair(k, bytes)) return e;
   const PairBwdArgs a{qkv,  ldq,    off,    sh.n_atoms, n0,  eb,   sh.slots, sh.heads,
                       sh.scale, dmerged, ldg, merged, ldm, ml, cf_seq, ldc, qkv_adj, lda, cfh, xf,
@@ -897,7 +942,9 @@ int pair_bwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
 }
 
-size_t pair_fwd_bytes(int HD, int NW) { return NW <= kPairMaxWaves ? PairFwdLds(HD, NW).bytes : ~size_t(0); }
+size_t pair_fwd_bytes(int HD, int NW) {
+  return NW <= kPairMaxWaves ? PairFwdLds(HD, pair_waves(NW)).bytes : ~size_t(0);
+}
 
 const void* pair_fwd_kernel_ptr(int HD) {
   return HD == 64 ? reinterpret_cast<const void*>(attn_fwd_pair_kernel<64, 5, false>)
@@ -906,7 +953,7 @@ const void* pair_fwd_kernel_ptr(int HD) {
 
 int pair_fwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* qkv, int64_t ldq, const int* off,
              const float* cf_seq, int64_t ldc, float* merged, int64_t ldm, float* ml, QkvXf xf, hipStream_t st) {
-  const int NW = (sh.slots + 15) / 16, HD = sh.head_dim;
+  const int NW = pair_waves((sh.slots + 15) / 16), HD = sh.head_dim;
   if (NW > kPairMaxWaves || (HD != 32 && HD != 64)) return PET_ATTN_ESLOTS;
   const int64_t items = int64_t(n1 - n0) * sh.heads;
   if (items == 0) return PET_ATTN_OK;
@@ -926,7 +973,12 @@ int pair_fwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
       case 5: pick(hd, std::integral_constant<int, 5>{}); break;
       case 6: pick(hd, std::integral_constant<int, 6>{}); break;
       case 7: pick(hd, std::integral_constant<int, 7>{}); break;
-      default: pick(hd, std::integral_constant<int, 8>{}); break;
+      case 8: pick(hd, std::integral_constant<int, 8>{}); break;
+      case 9: pick(hd, std::integral_constant<int, 9>{}); break;
+      case 10: pick(hd, std::integral_constant<int, 10>{}); break;
+      case 12: pick(hd, std::integral_constant<int, 12>{}); break;
+      case 14: pick(hd, std::integral_constant<int, 14>{}); break;
+      default: pick(hd, std::integral_constant<int, 16>{}); break;
     }
   };
   if (HD == 64)

@@ -125,6 +125,49 @@ def test_many_slots(device, hd, top):
     check_against_oracle(device, f"many slots hd {hd} S {tk.slots}", tk.off, tk.cf_seq, qkv, dm, 2, hd)
 
 
+@pytest.mark.parametrize("hd,S", [(32, 129), (32, 144), (32, 160), (32, 177), (32, 224), (32, 241), (32, 256), (64, 129),
+                                  (64, 160)])
+def test_pair_kernels_past_128_slots(device, hd, S):
+    # the fp16-pair kernels with more than eight waves, at the edges of every
+    # wave count (nine with unpadded rows, sixteen; waves left idle by the
+    # rounding to an even count and by shorter atoms)
+    plan = A._lib.describe(5, 4000, S, 2, hd)
+    assert plan["fwd_pair"] == 1 and plan["bwd_pair"] == 1, plan
+    counts = [S - 1, 0, S - 2, 15, 127, S // 2, 1, 128]
+    tk, qkv, dm = random_case(counts, 2, hd, seed=S, cf_kind="zeros")
+    assert tk.slots == S
+    check_against_oracle(device, f"pair kernels S {S} hd {hd}", tk.off, tk.cf_seq, qkv, dm, 2, hd)
+
+
+@pytest.mark.parametrize("S,hd", [(143, 32), (220, 32), (150, 64)])
+def test_op_level_block_pairs_past_128_slots(device, S, hd):
+    # qkv_adj as block pairs into the input adjoint's product, past eight
+    # waves: in_adj against the fp64 product of the core's qkv_adj (its pairs
+    # hold 22 bits, 2^-22 of each slice's largest value, plus the product's fp32
+    # accumulation over 3D: 1e-5 of the row's largest)
+    H, D, n = 8, 8 * hd, 2 ** 32 // (3 * (8 * hd) ** 2) // S + 2
+    say(f"[gpu] op level S {S} hd {hd} atoms {n}")
+    rng = np.random.default_rng(S)
+    tk = systems.tokens_from_counts(rng.integers(S // 2, S, n).tolist() + [S - 1], seed=S)
+    T, N = tk.n_rows, tk.n_atoms
+    q = torch.randn(T, 3 * D, device=device, generator=torch.Generator(device=device).manual_seed(S))
+    g = torch.randn(T, D, device=device, generator=torch.Generator(device=device).manual_seed(S + 1))
+    w_in, w_out = dev(rng.standard_normal((3 * D, D)) / D ** 0.5, device), torch.eye(D, device=device)
+    off, cf = dev(tk.off, device, torch.int32), dev(tk.cf_seq, device)
+    ws = A.Workspace(device)
+    out, in_adj = torch.empty(T, D, device=device), torch.empty(T, D, device=device)
+    ca = torch.zeros(N, tk.slots, device=device)
+    args = (A.Tokens(off, N), tk.slots, H, hd, 1.0)
+    A.attention(ws, "l", out, q, cf, w_out, None, *args, True)
+    A.attention_bwd(ws, "l", in_adj, ca, g, q, cf, w_in, w_out, *args, 0.0)
+    merged, ml = A.attn_fwd(q, off, cf, H, hd)
+    qa, ca2, _ = A.attn_bwd(q, off, g, merged, ml, cf, H, hd)
+    ref = qa.double() @ w_in.double()
+    err = ((in_adj - ref).abs() / ref.abs().amax(1, keepdim=True)).max().item()
+    assert err <= 1e-5, err
+    assert torch.allclose(ca, ca2, rtol=1e-4, atol=1e-4 * ca2.abs().max().item())
+
+
 def test_max_slots(device):
     # the LDS-staged kernels' envelope; past it (and for head_dims not a
     # multiple of 16) the streaming kernels run (tests/test_gpu_stream.py)
