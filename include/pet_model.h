@@ -163,11 +163,11 @@ PET_ATTN_API int pet_linear_fused_split_ws(int M, int N, int K, const float* A, 
  * W [N, K] given by pet_linear_pair_weights as rows of three fp16 parts (W's
  * rows each scaled by a power of two and split into hi, mid and lo, which sum
  * to it exactly; N * K * 6 + N * 4 bytes, 16-byte aligned), A fp32 (lda a
- * multiple of 4, 16-byte aligned), epilogue as pet_linear_fused. The weights
- * of a wave's output columns stay in its registers; a workgroup splits each
- * 16-row block of A into fp16 pairs once for its four waves and runs five part
- * products on the 16-bit matrix cores (all but a_lo b_lo), so a row's results
- * depend on that row alone (not on M or the tiling) and repeat bit for bit. No counterpart in
+ * multiple of 4, 16-byte aligned), epilogue as pet_linear_fused. A's rows are
+ * split into fp16 pairs as they are read, with five part products on the
+ * 16-bit matrix cores (all but a_lo b_lo), each step of 32 summed on its own, so a
+ * row's results depend on that row alone (not on M or the tiling) and repeat
+ * bit for bit. No counterpart in
  * the reference, which runs these layers in fp32 (src/fused_gemm_hip.cpp). */
 PET_ATTN_API int pet_linear_pair_weights(const float* W, int N, int K, int64_t ldw, void* out, void* stream);
 PET_ATTN_API int pet_linear_fused_smallk(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs,
@@ -226,7 +226,7 @@ PET_ATTN_API int pet_linear_fused_blocks(int M, int N, int K, const void* Ablock
  * have launched in this process, by the instructions that run them:
  * flops[0] the fp32 fused kernel (fp32 matrix cores), [1] split-fp32 as bf16
  * parts (six bf16 products each), [2] fp16 pairs (three fp16 products), [3]
- * the short-K kernel (five fp16 products); products on rocBLAS are not
+ * the three-part kernels (five fp16 products); products on rocBLAS are not
  * counted. reset != 0 zeroes the counts after reading them. A measurement aid
  * with no counterpart in the reference: the bench prices an evaluation's
  * products at the ceilings of the instructions that ran them. Counted at

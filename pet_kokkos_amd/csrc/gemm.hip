@@ -31,17 +31,15 @@
 #include <cstdlib>
 
 #include "../../include/pet_model.h"
+#include "gemm_common.h"
 #include "split_bf16.h"
 
 namespace pet_gemm {
 
-using pet_split::f4;
 using pet_split::mfma6;
 using pet_split::pack_hi;
 using pet_split::split3;
 using pet_split::split8;
-using pet_split::u4;
-using pet_split::u2;
 using pet_split::mfma3;
 using pet_split::mfma_h;
 using pet_split::pair2;
@@ -50,38 +48,7 @@ using pet_split::pair_scale;
 __device__ __forceinline__ f4 mfma(float a, float b, const f4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ float sig_fast(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
-
-struct Epi {
-  const float* row_scale = nullptr;  // [M]
-  const float* bias = nullptr;       // [N]
-  const float* cin = nullptr;        // [M, N] (ld ldcin), scaled by beta
-  int64_t ldcin = 0;
-  float beta = 0.f;
-  float* pre = nullptr;              // [M, N] (ld ldpre): v before the activation
-  int64_t ldpre = 0;
-  int act = 0;                       // 0 none, 1 SiLU, 2 SwiGLU (C has N/2 columns),
-                                     // 3 / 4 the backward of SiLU / SwiGLU (below)
-  // Block pairs in place of C (staged epilogue only): the output row i as
-  // fp16 pairs in pair_act_kernel's layout (kgo k groups of 8 a row, each
-  // group's hi then lo 16 bytes), scaled per (row, column tile) -- the tile's
-  // output columns are one K block of the product that reads them -- with the
-  // block's inverse scale at pinv[block ldinv + i].
-  u4* pout = nullptr;
-  float* pinv = nullptr;
-  int64_t ldinv = 0;
-  int kgo = 0;
-};
-
-// FLOPs (2 M N K) of the products this library's dense kernels have launched,
-// by the instructions that run them: 0 the fp32 fused kernel (fp32 matrix
-// cores), 1 split-fp32 as three bf16 parts (six bf16 products), 2 fp16 pairs
-// (three fp16 products), 3 the short-K kernel (five fp16 products). A
-// measurement aid, process-wide (pet_gemm_flop_tally).
 std::atomic<uint64_t> g_flops[4];
-inline void tally(int cls, int64_t M, int64_t N, int64_t K) {
-  g_flops[cls].fetch_add(uint64_t(2) * uint64_t(M) * uint64_t(N) * uint64_t(K), std::memory_order_relaxed);
-}
 
 // The epilogue of one result element v at (i, j), shared by the kernels. Every
 // lane of the wave calls it together (SwiGLU pairs neighbouring lanes):
@@ -822,37 +789,6 @@ __global__ void __launch_bounds__(256) pair_act_kernel(const float* __restrict__
   if (l == 0) reinterpret_cast<float*>(out + int64_t(M) * KG * 2)[row] = 1.f / s;
 }
 
-// The K loop's barrier: no memory fence, since any fence, even one on LDS
-// alone, makes the compiler wait for every global-to-LDS load in flight (the
-// prefetches too). The loop's own vmcnt wait before it covers the step's
-// loads; an explicit lgkmcnt(0) wait (vmcnt and expcnt left at their maxima)
-// makes every LDS read a wave issued in the step before complete before it
-// passes, so no wave's global_load_lds can overwrite a stage another is still
-// reading, whatever order the compiler gives the products; the empty asm
-// keeps the compiler from moving memory accesses across it.
-__device__ __forceinline__ void ring_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-
-// 16 bytes a lane from global memory into LDS, a wave's 64 lanes filling
-// dst .. dst + 1 KB in lane order (dst wave-uniform). A device function: the
-// builtin, called in a lambda of a kernel, stops the host side from emitting
-// the kernel.
-__device__ __forceinline__ void ring_load(const u4* src, u4* dst) {
-  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
-}
-
-// s_waitcnt on the vector-memory counter alone (gfx9 encoding: vmcnt in bits
-// 3:0 and 15:14; expcnt 7 and lgkmcnt 15 wait for nothing).
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
 // C = epi(A B^T) with both operands as fp16 pairs (pair_act_kernel's and
 // pair_rows_kernel's layout): a row's K step of 32 is 8 u4, part p = 2 group +
 // (0 hi, 1 lo). No vector arithmetic in the K loop: the steps go from global
@@ -1032,281 +968,6 @@ __attribute__((amdgpu_waves_per_eu(BM == 128 && BN == 128 ? 4 : 1))) gemm_pp_ker
   static_assert(ST * (BM + BN) * 128 >= BM * BN * 4, "the ring holds the result tile");
   if (staged_epilogue<BM, BN, WGM, WGN, 1, PO>(acc, reinterpret_cast<float*>(ring), m0, n0, M, N, C, ldc, epi)) return;
   if constexpr (!PO) epilogue<WM, WN>(acc, m0, n0, wm, wn, c, g, M, N, C, ldc, epi);  // (block pairs: the host makes sure of the staged one)
-}
-
-// epi_elem's arithmetic, in its order, for four consecutive output columns
-// j .. j + 3 of row i (j a multiple of 4; a SwiGLU pair in one lane), with
-// 16-byte accesses where vec (every pointer 16-byte aligned, every leading
-// dimension and N multiples of 4), element by element otherwise.
-template <bool vec, bool bwd>
-__device__ __forceinline__ void epi_quad(float (&v)[4], int i, int j, int M, int N, float* C, int64_t ldc,
-                                         const Epi& epi, const float4* bq = nullptr) {
-  if (i >= M || j >= N) return;
-  if constexpr (bwd) {
-    const float* z = epi.cin + int64_t(i) * epi.ldcin;
-    if constexpr (vec) {  // z, bias and C rows 16-byte aligned, N a multiple of 4
-      if (epi.act == 3) {
-        const float4 z4 = *reinterpret_cast<const float4*>(z + j);
-        const float4 b4 = epi.bias ? *reinterpret_cast<const float4*>(epi.bias + j) : make_float4(0.f, 0.f, 0.f, 0.f);
-        const float xs[4] = {z4.x + b4.x, z4.y + b4.y, z4.z + b4.z, z4.w + b4.w};
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float sg = sig_fast(xs[e]);
-          o[e] = v[e] * (sg * (1.0f + xs[e] * (1.0f - sg)));
-        }
-        *reinterpret_cast<float4*>(C + int64_t(i) * ldc + j) = make_float4(o[0], o[1], o[2], o[3]);
-      } else {  // (value, gate) pairs 2 j .. 2 j + 7
-        float zz[8];
-        *reinterpret_cast<float4*>(zz) = *reinterpret_cast<const float4*>(z + 2 * j);
-        *reinterpret_cast<float4*>(zz + 4) = *reinterpret_cast<const float4*>(z + 2 * j + 4);
-        if (epi.bias) {
-          const float4 b0 = *reinterpret_cast<const float4*>(epi.bias + 2 * j);
-          const float4 b1 = *reinterpret_cast<const float4*>(epi.bias + 2 * j + 4);
-          zz[0] += b0.x, zz[1] += b0.y, zz[2] += b0.z, zz[3] += b0.w;
-          zz[4] += b1.x, zz[5] += b1.y, zz[6] += b1.z, zz[7] += b1.w;
-        }
-        float o[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float u = zz[2 * e], sg = sig_fast(zz[2 * e + 1]);
-          o[2 * e] = v[e] * sg;
-          o[2 * e + 1] = v[e] * u * sg * (1.0f - sg);
-        }
-        float* cr = C + int64_t(i) * ldc + 2 * j;
-        *reinterpret_cast<float4*>(cr) = make_float4(o[0], o[1], o[2], o[3]);
-        *reinterpret_cast<float4*>(cr + 4) = make_float4(o[4], o[5], o[6], o[7]);
-      }
-      return;
-    }
-    if (epi.act == 3) {
-      float o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (!vec && j + e >= N) break;
-        const float x = z[j + e] + (epi.bias ? epi.bias[j + e] : 0.f), sg = sig_fast(x);
-        o[e] = v[e] * (sg * (1.0f + x * (1.0f - sg)));
-        if (!vec) C[int64_t(i) * ldc + j + e] = o[e];
-      }
-      if (vec) *reinterpret_cast<float4*>(C + int64_t(i) * ldc + j) = make_float4(o[0], o[1], o[2], o[3]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (j + e >= N) break;
-        const int jj = j + e;
-        const float u = z[2 * jj] + (epi.bias ? epi.bias[2 * jj] : 0.f);
-        const float sg = sig_fast(z[2 * jj + 1] + (epi.bias ? epi.bias[2 * jj + 1] : 0.f));
-        *reinterpret_cast<float2*>(C + int64_t(i) * ldc + 2 * jj) = make_float2(v[e] * sg, v[e] * u * sg * (1.0f - sg));
-      }
-    }
-    return;
-  }
-  const int ne = vec ? 4 : min(4, N - j);
-  if (epi.row_scale) {
-    const float rs = epi.row_scale[i];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] *= rs;
-  }
-  if (epi.bias) {
-    if (vec) {
-      const float4 b4 = bq ? *bq : *reinterpret_cast<const float4*>(epi.bias + j);
-      v[0] += b4.x, v[1] += b4.y, v[2] += b4.z, v[3] += b4.w;
-    } else {
-      for (int e = 0; e < ne; ++e) v[e] += epi.bias[j + e];
-    }
-  }
-  if (epi.cin) {
-    const float* ci = epi.cin + int64_t(i) * epi.ldcin + j;
-    if (vec) {
-      const float4 c4 = *reinterpret_cast<const float4*>(ci);
-      v[0] += epi.beta * c4.x, v[1] += epi.beta * c4.y, v[2] += epi.beta * c4.z, v[3] += epi.beta * c4.w;
-    } else {
-      for (int e = 0; e < ne; ++e) v[e] += epi.beta * ci[e];
-    }
-  }
-  if (epi.pre) {
-    float* pr = epi.pre + int64_t(i) * epi.ldpre + j;
-    if (vec) {
-      *reinterpret_cast<float4*>(pr) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-      for (int e = 0; e < ne; ++e) pr[e] = v[e];
-    }
-  }
-  float* ci = C + int64_t(i) * ldc;
-  if (epi.act == 2) {  // N even: pairs (j, j + 1), (j + 2, j + 3)
-    const float o0 = v[0] * sig_fast(v[1]), o1 = v[2] * sig_fast(v[3]);
-    if (vec) {
-      *reinterpret_cast<float2*>(ci + j / 2) = make_float2(o0, o1);
-    } else {
-      ci[j / 2] = o0;
-      if (ne > 2) ci[j / 2 + 1] = o1;
-    }
-    return;
-  }
-  if (epi.act == 1) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = v[e] * sig_fast(v[e]);
-  }
-  if (vec) {
-    *reinterpret_cast<float4*>(ci + j) = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    for (int e = 0; e < ne; ++e) ci[j + e] = v[e];
-  }
-}
-
-// Small K (at most 128), weights in registers. A workgroup of four waves
-// owns four groups of 16 TN output columns, one a wave, each holding its
-// columns' weights as three fp16 parts in registers (loaded once, TN KB 12
-// registers), and streams 16-row blocks of A: per block each thread takes one
-// k group of 8 (a row's groups in KL consecutive lanes, KL the power of two at
-// or above K / 8), the row's largest |x| comes from a shuffle over those
-// lanes, and the rows are split into fp16 pairs once for the workgroup into a
-// double-buffered LDS slice (rows padded to an odd number of 16-byte slots, so
-// that the 16 rows a fragment read meets fall on distinct banks); the thread
-// then loads its group of the next block into the registers it has just read.
-// After one barrier each wave reads its operand fragments and runs the five
-// part products per k group (a_hi and a_lo against w_hi and w_mid, and a_hi
-// w_lo; the dropped a_lo w_lo is below 2^-33 of |a||w|), the column tiles'
-// accumulations interleaved, with the weights as the instruction's first
-// operand: lane (c, g) then holds output row c, columns 4 g .. 4 g + 3 of
-// each 16-column tile, and the epilogue reads and writes 16 bytes a lane.
-// XCD x (workgroup L on x = L mod 8) takes rows [x M / 8, (x + 1) M / 8) in S
-// ranges per set of four column groups, so the sets re-read a range of A
-// from their XCD's L2. A row's results depend on that row alone, and the
-// products are summed in the order of the LDS-staged kernel this replaced:
-// the same bits.
-template <int KB, int TN, bool VEC, bool BWD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TN * KB <= 2 ? 4 : TN * KB <= 4 && !BWD ? 3 : 2)))
-gemm_skt_kernel(int M, int N, const float* __restrict__ A, int64_t lda, const u4* __restrict__ Bp, float* C,
-                int64_t ldc, Epi epi, int S) {
-  // RB 16-row tiles a block (2, with twice the rows in flight, crashes the
-  // ROCm 7.2 compiler's copy propagation at K = 128)
-  constexpr int RB = 1;
-  constexpr int KG = 4 * KB, CW = 16 * TN, RP = 2 * KG + 1, NW = 4, T = 64 * NW, R = 16 * RB;
-  __shared__ u4 sa[2][R * RP];
-  __shared__ float sinv[2][R];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
-  const int CG = (N + CW - 1) / CW, CS = (CG + NW - 1) / NW, x = blockIdx.x % 8, li = blockIdx.x / 8;
-  if (li >= CS * S) return;  // (uniform over the workgroup)
-  const int cs = li % CS, rs = li / CS, cg = cs * NW + w, n0 = cg * CW;
-  const bool live = cg < CG;  // a wave past the last column group still splits rows for the others
-  const int xr0 = int(int64_t(x) * M / 8), xr1 = int(int64_t(x + 1) * M / 8);
-  const int nb = (xr1 - xr0 + R - 1) / R;
-  const int b0 = int(int64_t(rs) * nb / S), b1 = int(int64_t(rs + 1) * nb / S);
-  if (b0 >= b1) return;  // (uniform)
-  u4 wh[TN][KB], wm[TN][KB], wl[TN][KB];
-  float ib[TN][4];
-  {
-    const float* inv_b = reinterpret_cast<const float*>(Bp + int64_t(N) * KG * 3);
-#pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      const u4* br = Bp + int64_t(min(n0 + 16 * b + c, N - 1)) * (3 * KG);
-#pragma unroll
-      for (int kk = 0; kk < KB; ++kk) {
-        wh[b][kk] = br[(4 * kk + g) * 3];
-        wm[b][kk] = br[(4 * kk + g) * 3 + 1];
-        wl[b][kk] = br[(4 * kk + g) * 3 + 2];
-      }
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) ib[b][rr] = inv_b[min(n0 + 16 * b + 4 * g + rr, N - 1)];
-    }
-  }
-  constexpr bool HB = VEC && !BWD;  // a forward epilogue with 16-byte accesses: the bias held
-  float4 bq[HB ? TN : 1];
-  if constexpr (HB) {
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-      bq[b] = epi.bias && live ? *reinterpret_cast<const float4*>(epi.bias + min(n0 + 16 * b + 4 * g, N - 4))
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  // a thread's k groups of a block: item e = tid + T q, row e / KL, group
-  // e % KL (KL the power of two at or above KG: a row's groups are KL
-  // consecutive lanes of one wave, those at KG and above idle); loaded one
-  // block ahead, into the registers the split has just read
-  constexpr int KL = KG <= 4 ? 4 : KG <= 8 ? 8 : 16, ITEMS = R * KL, NI = (ITEMS + T - 1) / T;
-  static_assert(ITEMS % T == 0 || ITEMS < T, "whole passes");
-  float4 v0[NI], v1[NI];
-  auto load_a = [&](int blk) {
-#pragma unroll
-    for (int q = 0; q < NI; ++q) {
-      const int e = tid + T * q;
-      if (e < ITEMS && e % KL < KG) {
-        const float* p = A + int64_t(min(xr0 + R * blk + e / KL, xr1 - 1)) * lda + 8 * (e % KL);
-        v0[q] = *reinterpret_cast<const float4*>(p);
-        v1[q] = *reinterpret_cast<const float4*>(p + 4);
-      } else {
-        v0[q] = v1[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    }
-  };
-  load_a(b0);
-  for (int blk = b0; blk < b1; ++blk) {
-    const int buf = (blk - b0) & 1;
-#pragma unroll
-    for (int q = 0; q < NI; ++q) {
-      const int e = tid + T * q, ir = e / KL, ij = e % KL;
-      float m = fmaxf(fmaxf(fmaxf(fabsf(v0[q].x), fabsf(v0[q].y)), fmaxf(fabsf(v0[q].z), fabsf(v0[q].w))),
-                      fmaxf(fmaxf(fabsf(v1[q].x), fabsf(v1[q].y)), fmaxf(fabsf(v1[q].z), fabsf(v1[q].w))));
-#pragma unroll
-      for (int o = 1; o < KL; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));  // the row's KL consecutive lanes
-      const float sc = pair_scale(m);
-      unsigned h[4], lo[4];
-      pair2(v0[q].x * sc, v0[q].y * sc, h[0], lo[0]);
-      pair2(v0[q].z * sc, v0[q].w * sc, h[1], lo[1]);
-      pair2(v1[q].x * sc, v1[q].y * sc, h[2], lo[2]);
-      pair2(v1[q].z * sc, v1[q].w * sc, h[3], lo[3]);
-      if (e < ITEMS && ij < KG) {
-        sa[buf][ir * RP + 2 * ij] = u4{h[0], h[1], h[2], h[3]};
-        sa[buf][ir * RP + 2 * ij + 1] = u4{lo[0], lo[1], lo[2], lo[3]};
-        if (ij == 0) sinv[buf][ir] = 1.f / sc;
-      }
-    }
-    load_a(min(blk + 1, b1 - 1));  // (the last block's rows again at the end: in bounds, unused)
-    __syncthreads();  // the block's pairs are in LDS; (double buffer) no wave still reads the slice two blocks back
-    if (live) {
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        u4 ah[KB], al[KB];
-#pragma unroll
-        for (int kk = 0; kk < KB; ++kk) {
-          ah[kk] = sa[buf][(16 * r + c) * RP + 2 * (4 * kk + g)];
-          al[kk] = sa[buf][(16 * r + c) * RP + 2 * (4 * kk + g) + 1];
-        }
-        const float isc = sinv[buf][16 * r + c];
-        const int i = xr0 + R * blk + 16 * r + c;
-        // the tiles' chains interleaved (each tile's products in the same
-        // order, small ones first), so TN independent accumulations are in
-        // flight
-        f4 acc[TN];
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[b] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < KB; ++kk) {
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[b] = pet_split::mfma_h(wm[b][kk], al[kk], acc[b]);
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[b] = pet_split::mfma_h(wl[b][kk], ah[kk], acc[b]);
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[b] = pet_split::mfma_h(wh[b][kk], al[kk], acc[b]);
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[b] = pet_split::mfma_h(wm[b][kk], ah[kk], acc[b]);
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[b] = pet_split::mfma_h(wh[b][kk], ah[kk], acc[b]);
-        }
-#pragma unroll
-        for (int b = 0; b < TN; ++b) {
-          float o[4];
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) o[rr] = acc[b][rr] * isc * ib[b][rr];
-          if (i < xr1)
-            epi_quad<VEC, BWD>(o, i, n0 + 16 * b + 4 * g, M, N, C, ldc, epi, HB ? &bq[HB ? b : 0] : nullptr);
-          // (one tile's epilogue at a time: its loads are not hoisted above
-          // the last tile's stores, which would hold every tile's operands)
-          asm volatile("" ::: "memory");
-        }
-      }
-    }
-  }
 }
 
 }  // namespace pet_gemm
@@ -1755,53 +1416,6 @@ int pet_gemm_pair_weights(const float* W, int N, int K, int64_t ldw, bool transp
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
 }
 
-// C = epi(A B^T) for K at most 128 (a multiple of 32), B as rows of three
-// fp16 parts (pet_gemm_pair_weights): gemm_skt_kernel.
-int pet_gemm_nt_sk(int M, int N, int K, const float* A, int64_t lda, const void* Bp, float* C, int64_t ldc,
-                   const Epi& e, hipStream_t st) {
-  if (M < 0 || N < 0 || K < 32 || K > 128 || K % 32) return PET_ATTN_EINVAL;
-  if (M == 0 || N == 0) return PET_ATTN_OK;
-  if (lda % 4 || (reinterpret_cast<uintptr_t>(A) & 15) || (reinterpret_cast<uintptr_t>(Bp) & 15))
-    return PET_ATTN_EALIGN;
-  // 32 columns a wave (64 at K <= 64, where the weights take half the
-  // registers); about 64 workgroups an XCD (two a CU), the XCD's rows split
-  // into S ranges per set of four column groups. Measured on MI355X at
-  // 27318 rows (K 128, N 1024: 58 us against 78 for a 64 x 64-tile kernel
-  // staging the weights through LDS; 32 and 128 workgroups an XCD slower).
-  const int KB = K / 32, TN = KB <= 2 ? 4 : 2, CW = 16 * TN;
-  const int64_t CG = (N + CW - 1) / CW, CS = (CG + 3) / 4;
-  const int64_t rows_x = (M + 7) / 8, nbx = (rows_x + 15) / 16;
-  const int64_t S = std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>(1, 64 / CS), nbx));
-  const int64_t wgx = CS * S;
-  if (wgx * 8 >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
-  auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  const bool vec = N % 4 == 0 && a16(C) && ldc % 4 == 0 && (!e.bias || a16(e.bias)) &&
-                   (!e.cin || (a16(e.cin) && e.ldcin % 4 == 0)) && (!e.pre || (a16(e.pre) && e.ldpre % 4 == 0));
-  const u4* B = static_cast<const u4*>(Bp);
-  const dim3 grid{unsigned(wgx * 8)}, block{256};
-#define PET_SKT_LAUNCH(kb, tn, v, bw) \
-  hipLaunchKernelGGL((gemm_skt_kernel<kb, tn, v, bw>), grid, block, 0, st, M, N, A, lda, B, C, ldc, e, int(S))
-#define PET_SKT_GO(kb, tn)                    \
-  if (e.act >= 3 && vec)                      \
-    PET_SKT_LAUNCH(kb, tn, true, true);       \
-  else if (e.act >= 3)                        \
-    PET_SKT_LAUNCH(kb, tn, false, true);      \
-  else if (vec)                               \
-    PET_SKT_LAUNCH(kb, tn, true, false);      \
-  else                                        \
-    PET_SKT_LAUNCH(kb, tn, false, false)
-  switch (KB) {
-    case 1: PET_SKT_GO(1, 4); break;
-    case 2: PET_SKT_GO(2, 4); break;
-    case 3: PET_SKT_GO(3, 2); break;
-    default: PET_SKT_GO(4, 2); break;
-  }
-#undef PET_SKT_GO
-#undef PET_SKT_LAUNCH
-  tally(3, M, N, K);
-  return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
-}
-
 extern "C" int pet_linear_pair_weights(const float* W, int N, int K, int64_t ldw, void* out, void* stream) {
   if (N < 0 || K < 0 || K % 32 || ldw < K || ((N > 0 && K > 0) && (!W || !out))) return PET_ATTN_EINVAL;
   if (reinterpret_cast<uintptr_t>(out) & 15) return PET_ATTN_EALIGN;
@@ -1818,7 +1432,8 @@ extern "C" int pet_linear_fused_smallk(int M, int N, int K, const float* A, int6
   Epi e;
   e.row_scale = row_scale, e.bias = bias, e.cin = cin, e.ldcin = ldcin, e.beta = beta, e.pre = pre, e.ldpre = ldpre;
   e.act = act;
-  return pet_gemm_nt_sk(M, N, K, A, lda, Wpairs, C, ldc, e, reinterpret_cast<hipStream_t>(stream));
+  if (K > 128) return PET_ATTN_EINVAL;
+  return pet_gemm_nt_p3(M, N, K, A, lda, Wpairs, C, ldc, e, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int pet_linear_pair_rows(const float* X, int M, int K, int64_t ldx, void* out, void* stream) {

@@ -63,9 +63,10 @@ int pet_gemm_nt_pp_blocks(int M, int N, int K, const void* Ap, int kb, const voi
                           const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
                           float* pre, int64_t ldpre, int act, hipStream_t st);
 
-extern "C" int pet_linear_fused_smallk(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs, float* C,
-                                       int64_t ldc, const float* row_scale, const float* bias, const float* cin,
-                                       int64_t ldcin, float beta, float* pre, int64_t ldpre, int act, void* stream);
+// gemm_rows.hip: from weights in three exact fp16 parts (pet_gemm_pair_weights)
+int pet_gemm_nt_parts(int M, int N, int K, const float* A, int64_t lda, const void* Bp, float* C, int64_t ldc,
+                      const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
+                      float* pre, int64_t ldpre, int act, hipStream_t st);
 int pet_gemm_pair_weights(const float* W, int N, int K, int64_t ldw, bool transposed, void* out, hipStream_t st);
 
 namespace pet_model_impl {
@@ -570,7 +571,7 @@ struct pet_model {
   int tier = 1;                // the memory tier of the last evaluation: 1 never, 2 wide
   std::unordered_map<std::string, Mat> m;
   std::unordered_map<const float*, const void*> split;  // a matrix's split-row copy (K a multiple of 32)
-  std::unordered_map<const float*, const void*> psplit;  // its fp16 part rows at K <= 128 (the short-K kernel)
+  std::unordered_map<const float*, const void*> psplit;  // and its rows of three exact fp16 parts
   // layers whose saved pre-activation holds its bias (made by the split-product
   // kernel's epilogue in the forward in progress), read by their backward
   std::unordered_map<std::string, bool> pre_biased;
@@ -618,43 +619,33 @@ bool own_gemm(const pet_model& md, int M, int K) {
   return K % 16 == 0 && (md.gemm_mode == 1 || (md.gemm_mode == 2 && M <= 4096));
 }
 
-// out[M, N] = in W^T + beta out, W a model matrix [N, K]: rocBLAS fp32, or
-// this library's kernels where W has a copy in their form and in is 16-byte
-// aligned rows. By PET_OPT_MODEL_GEMM: 6 (the default) the split-product
-// kernel for the large products (M N K >= 2^32), the short-K kernel
-// (pet_linear_fused_smallk: the weights exact in three fp16 parts, A's rows
-// as fp16 pairs, five part products) for the K <= 128 products with a bias or
-// activation and N >= 64, rocBLAS for the rest; 4 as 6 without the short-K
-// kernel; 5 every product on this library's kernels -- the short-K kernel for
-// K at most 128, the split-product kernel above -- so that no result depends
-// on how many rows come with it and every bias and activation rides in an
-// epilogue; 3 the split-product kernel for every product; 0 rocBLAS only.
-// Measured on MI355X (energy+forces, ms): C2 2.585 / 1.92 (residual) with
-// mode 6, 2.80 / 2.07 with mode 4 (no C2 product is large), 2.89 / 1.95 with
-// mode 5, 3.59 / 2.40 with mode 3; C5 171 with mode 4, 170 with mode 5.
-// Energies from the float64 oracle, C2 / residual: mode 6 3.0e-7 / 3.8e-7,
-// mode 4 0.7e-7 / 4.2e-7, mode 5 1.5e-7 / 8.3e-7 (the float32 oracle 3.3e-7 /
-// 4.2e-7). The narrow products (N < 64: the readout's) stay off the short-K
-// kernel: its matrix instruction truncates each product toward zero below the
+// out[M, N] = in W^T + beta out, W a model matrix [N, K]: this library's
+// kernels where W has a copy in their form and in is 16-byte aligned rows, or
+// rocBLAS fp32. By PET_OPT_MODEL_GEMM: 6 (the default) the split-product kernel
+// for the large products past K = 128 (M N K >= 2^32), the three-part kernels
+// (pet_gemm_nt_parts: the weights exact in three fp16 parts, A's rows as fp16
+// pairs, five part products) for the rest with N >= 64, rocBLAS for the
+// narrow ones; 4 the split-product kernel for the large products, rocBLAS for
+// the rest; 5 every product on this library's kernels -- the three-part kernels
+// for K at most 128, the split-product kernel above -- so that no result depends
+// on how many rows come with it; 3 the split-product kernel for every product;
+// 0 rocBLAS only. The narrow products (N < 64: the readout's) stay on rocBLAS in
+// mode 6: the matrix instruction truncates each product toward zero below the
 // result's last place, and with a fixed weight vector and mostly positive
 // inputs those truncations share a sign on every atom and add up over a
 // structure (C2-residual 5.7e-7 with them on it).
 // The kernel a product takes (null: rocBLAS): the copy of W it reads and
-// whether it is the short-K kernel.
+// whether that is the three-part one.
 struct Sel {
   const void* p = nullptr;
-  bool sk = false;
+  bool parts = false;
   explicit operator bool() const { return p != nullptr; }
 };
-// fuse: the call has a bias or an activation for the epilogue (mode 6 takes
-// the short-K kernel for those products at K <= 128 and N >= 64, where it
-// saves a pass).
-Sel split_for(const pet_model& md, const float* in, int64_t ldi, const float* W, int M, int N, int K,
-              bool fuse = false) {
+Sel split_for(const pet_model& md, const float* in, int64_t ldi, const float* W, int M, int N, int K) {
   const int mode = md.gemm_mode;
   const bool big = double(M) * N * K >= 4294967296.0;
   if (ldi % 4 || (reinterpret_cast<uintptr_t>(in) & 15)) return {};
-  if ((mode == 5 || (mode == 6 && fuse && N >= 64)) && K <= 128 && K % 32 == 0) {
+  if (mode == 5 ? K <= 128 : mode == 6 && N >= 64 && (K <= 128 || !big)) {
     auto it = md.psplit.find(W);
     if (it != md.psplit.end()) return {it->second, true};
   }
@@ -668,9 +659,8 @@ Sel split_for(const pet_model& md, const float* in, int64_t ldi, const float* W,
 int own_nt(const pet_model& md, const Sel& sel, int M, int N, int K, const float* in, int64_t ldi, float* C,
            int64_t ldc, const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
            float* pre, int64_t ldpre, int act, hipStream_t st) {
-  if (sel.sk)
-    return pet_linear_fused_smallk(M, N, K, in, ldi, sel.p, C, ldc, row_scale, bias, cin, ldcin, beta, pre, ldpre,
-                                   act, st);
+  if (sel.parts)
+    return pet_gemm_nt_parts(M, N, K, in, ldi, sel.p, C, ldc, row_scale, bias, cin, ldcin, beta, pre, ldpre, act, st);
   return pet_gemm_nt_split(M, N, K, in, ldi, sel.p, C, ldc, row_scale, bias, cin, ldcin, beta, pre, ldpre, act, st,
                            md.pairs, md.pairs ? md.kPairsBytes : 0);
 }
@@ -693,7 +683,7 @@ void linear(pet_model& md, float* out, const float* in, int M, int K, const std:
     ok(pet_gemm_nt_fused(M, W.rows, K, in, K, W.p, K, out, W.rows, nullptr, b, nullptr, 0, 0.f, nullptr, 0, 0, st));
     return;
   }
-  if (const Sel sp = split_for(md, in, K, W.p, M, W.rows, K, b != nullptr)) {  // the bias in the epilogue
+  if (const Sel sp = split_for(md, in, K, W.p, M, W.rows, K)) {  // the bias in the epilogue
     ok(own_nt(md, sp, M, W.rows, K, in, K, out, W.rows, nullptr, b, nullptr, 0, 0.f, nullptr, 0, 0, st));
     return;
   }
@@ -725,7 +715,7 @@ void linear_acc_bias(pet_model& md, float* out, const float* in, int M, int K, c
   const Mat& W = md.w(key + ".weight");
   if (W.cols != K) throw Error{PET_MODEL_ESHAPE};
   if (M == 0) return;
-  if (const Sel sp = own_gemm(md, M, K) ? Sel{} : split_for(md, in, K, W.p, M, W.rows, K, true)) {
+  if (const Sel sp = own_gemm(md, M, K) ? Sel{} : split_for(md, in, K, W.p, M, W.rows, K)) {
     ok(own_nt(md, sp, M, W.rows, K, in, K, out, W.rows, nullptr, md.p(key + ".bias"), out, W.rows, 1.f, nullptr, 0, 0,
               st));
     return;
@@ -750,7 +740,7 @@ const float* pass_bias(const pet_model& md, const std::string& key);
 bool linear_bwd_act(pet_model& md, float* out, const float* adj, int M, const std::string& key_out, const float* z,
                     const std::string& key_act, int act, hipStream_t st) {
   const Mat& WT = md.w(key_out + ".weight^T");
-  const Sel sp = M ? split_for(md, adj, WT.cols, WT.p, M, WT.rows, WT.cols, true) : Sel{};
+  const Sel sp = M ? split_for(md, adj, WT.cols, WT.p, M, WT.rows, WT.cols) : Sel{};
   if (!sp) return false;
   const int64_t w = act == 2 ? 2 * int64_t(WT.rows) : WT.rows;
   ok(own_nt(md, sp, M, WT.rows, WT.cols, adj, WT.cols, out, w, nullptr, pass_bias(md, key_act), z, w, 0.f, nullptr, 0,
@@ -776,14 +766,14 @@ void linear_pre(pet_model& md, float* z, const float* in, int M, int K, const st
 // Whether linear_act fuses the layer (then out must be a buffer other than in).
 bool act_fuses(const pet_model& md, const float* in, int M, int K, const std::string& key) {
   const Mat& W = md.w(key + ".weight");
-  return !own_gemm(md, M, K) && bool(split_for(md, in, K, W.p, M, W.rows, K, true));
+  return !own_gemm(md, M, K) && bool(split_for(md, in, K, W.p, M, W.rows, K));
 }
 bool linear_act(pet_model& md, float* out, float* z, const float* in, int M, int K, const std::string& key, int act,
                 hipStream_t st) {
   const Mat& W = md.w(key + ".weight");
   if (W.cols != K) throw Error{PET_MODEL_ESHAPE};
   // (out must not be the GEMM's input: other workgroups still read its rows)
-  const Sel sp = own_gemm(md, M, K) || out == in ? Sel{} : split_for(md, in, K, W.p, M, W.rows, K, true);
+  const Sel sp = own_gemm(md, M, K) || out == in ? Sel{} : split_for(md, in, K, W.p, M, W.rows, K);
   md.pre_biased[key] = bool(sp);
   if (!sp || M == 0) return false;
   ok(own_nt(md, sp, M, W.rows, K, in, K, out, act == 2 ? W.rows / 2 : W.rows, nullptr, md.p(key + ".bias"), nullptr, 0,
@@ -1795,11 +1785,11 @@ int pet_model_create(const pet_model_hypers* hy, const pet_model_tensor* tensors
       }
       if (hipDeviceSynchronize() != hipSuccess) throw Error{PET_ATTN_ELAUNCH};
     }
-    // the matrices with K at most 128 as rows of three fp16 parts, for the short-K kernel
+    // and as rows of three fp16 parts, for the three-part kernels
     std::vector<std::pair<const Mat*, size_t>> pat;
     size_t ptotal = 0;
     for (auto& [n, mt] : md->m)
-      if (mt.cols > 0 && mt.cols <= 128 && mt.cols % 32 == 0)
+      if (mt.cols > 0 && mt.cols % 32 == 0)
         pat.push_back({&mt, ptotal}), ptotal += (size_t(6) * mt.rows * mt.cols + size_t(4) * mt.rows + 255) & ~size_t(255);
     if (ptotal) {
       if (hipMalloc(&md->wpair, ptotal) != hipSuccess) throw Error{PET_MODEL_EMEMORY};

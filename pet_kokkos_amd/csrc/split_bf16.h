@@ -122,6 +122,12 @@ __device__ __forceinline__ float pair_scale(float m) {
   const int e = __builtin_amdgcn_frexp_expf(m);
   return __builtin_amdgcn_ldexpf(1.f, min(15 - e, 126));
 }
+// pair_scale for one of several K blocks of a row, whose scales the product
+// that reads them compares: a block of zeros takes the largest scale, so that it
+// never sets the row's.
+__device__ __forceinline__ float block_scale(float m) {
+  return m > 0.f ? pair_scale(m) : __builtin_amdgcn_ldexpf(1.f, 126);
+}
 
 // The same pairs on the 16 x 16 x 16 instruction (k = 16: four fp16 values a
 // lane, two registers), for products whose contraction is one 16-row block.

@@ -588,3 +588,61 @@ def test_flop_tally(device):
     assert t["shortk"] == 2.0 * M * N * K and t["fp32"] == 2.0 * M * N * K
     assert t["split"] == 0.0 and t["pair"] == 0.0
     assert all(v == 0.0 for v in _lib.gemm_flop_tally().values())
+
+
+# the strip (M N from 3 * 2^20: partial strips of 128 and of 64 columns, one to four
+# steps of 32), 64 x 128, 64 x 64 and 32 x 64 tiles, and per-element epilogues
+@pytest.mark.parametrize("M,N,K", [(25001, 136, 128), (13107, 256, 96), (100003, 36, 32), (50021, 66, 64),
+                                   (32777, 68, 128), (8191, 260, 128), (701, 72, 64), (17, 33, 32)])
+def test_three_part_kernels(M, N, K, device):
+    """The short-K layer's kernels over their dispatch, with rows over 40
+    octaves, rows that outgrow their first 32 values by up to 2^20 (the running
+    scale), zero rows, and every epilogue. An element's error is bounded by
+    2^-20 of sum |a| |w|: the rows' pairs hold 24 bits less a half (2^-24), each
+    step's five instructions round by at most 2^-23 of the step's magnitudes, the
+    steps' sums by 2^-24 each; the weights are exact. A row alone gives the bits
+    it has among the others, whichever kernel takes either product."""
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    A = torch.randn(M, K, device=device, generator=g) * torch.exp2(
+        torch.randint(-20, 21, (M, 1), device=device, generator=g).float())
+    A[3::7, K // 2:] *= torch.exp2(torch.randint(0, 21, (A[3::7].shape[0], 1), device=device, generator=g).float())
+    A[1::11] = 0
+    W = torch.randn(N, K, device=device, generator=g) / K ** 0.5
+    b = torch.randn(N, device=device, generator=g)
+    P = L.PairWeights(W)
+    ref = A.double() @ W.double().T
+    bound = 2.0 ** -20 * (A.double().abs() @ W.double().abs().T)
+    C, pre = torch.full((M, N), float("nan"), device=device), torch.full((M, N), float("nan"), device=device)
+    L.fused(A, P, C)
+    assert ((C.double() - ref).abs() <= bound).all()
+    z = ref + b.double()
+    L.fused(A, P, C, bias=b, pre=pre, act=1)
+    tol = bound + 2.0 ** -22 * z.abs()  # the bias's sum
+    assert ((pre.double() - z).abs() <= tol).all()
+    # silu' is at most 1.1; sigmoid to 2^-20 of itself, and to 1e-37 where it is less
+    assert ((C.double() - z * torch.sigmoid(z)).abs() <= 1.1 * tol + 2.0 ** -20 * (z * torch.sigmoid(z)).abs()
+            + 1e-30 * z.abs()).all()
+    x = torch.randn(M, N, device=device, generator=g)
+    sg = torch.sigmoid(x.double())
+    L.fused(A, P, C, cin=x, act=3)
+    d = sg * (1 + x.double() * (1 - sg))
+    assert ((C.double() - ref * d).abs() <= (bound + 2.0 ** -20 * ref.abs()) * 1.5).all()
+    x2 = torch.randn(M, 2 * N, device=device, generator=g)
+    u, s2 = x2.double()[:, ::2], torch.sigmoid(x2.double()[:, 1::2])
+    C4 = torch.full((M, 2 * N), float("nan"), device=device)
+    L.fused(A, P, C4, cin=x2, act=4)
+    r4 = torch.stack([ref * s2, ref * u * s2 * (1 - s2)], -1).reshape(M, 2 * N)
+    f4 = torch.stack([torch.ones_like(u), u.abs().clamp(min=1)], -1).reshape(M, 2 * N)
+    tol4 = (bound + 2.0 ** -20 * ref.abs()).repeat_interleave(2, 1) * f4
+    assert ((C4.double() - r4).abs() <= tol4).all()
+    cin = x.clone()
+    L.fused(A, P, cin, bias=b, cin=cin, beta=0.5)  # the residual in place
+    assert ((cin.double() - (z + 0.5 * x.double())).abs() <= tol + 2.0 ** -22 * x.double().abs()).all()
+    if N % 2 == 0:
+        H = torch.full((M, N // 2), float("nan"), device=device)
+        L.fused(A, P, H, bias=b, pre=pre, act=2)
+        lo, hi = M // 3, min(M, M // 3 + 70)
+        H2, pre2 = torch.empty(hi - lo, N // 2, device=device), torch.empty(hi - lo, N, device=device)
+        L.fused(A[lo:hi].clone(), P, H2, bias=b, pre=pre2, act=2)
+        assert torch.equal(H[lo:hi], H2) and torch.equal(pre[lo:hi], pre2)
+        assert ((pre.double() - z).abs() <= tol).all()
