@@ -543,7 +543,7 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[t][e] = acc[t][e] * f3[m], mx = fmaxf(mx, fabsf(v[t][e]));
-      const float s = pet_split::pair_scale(max_g(mx));
+      const float s = pet_split::block_scale(max_g(mx));
       // lanes g and g ^ 1 (lanes l and l ^ 16) hold the two halves of the
       // 8-value groups 2t + g / 2: the even lane writes the group of each even
       // t, the odd lane that of each odd t, each trading the float4 the other

@@ -108,7 +108,7 @@ __device__ __forceinline__ void epilogue(const f4 (&acc)[WM / 16][WN / 16], int 
 // stores to four rows. False (nothing written) where a pointer or leading
 // dimension does not allow the 16-byte accesses; the caller then uses
 // epilogue(). tile: BM BN floats of LDS no wave still reads.
-template <int BM, int BN, int WGM, int WGN, int PASSES = 1, bool PO = false>
+template <int BM, int BN, int WGM, int WGN, int PASSES = 1>
 __device__ __forceinline__ bool staged_epilogue(const f4 (&acc)[BM / WGM / 16][BN / WGN / 16], float* tile, int m0,
                                                 int n0, int M, int N, float* C, int64_t ldc, const Epi& epi) {
   constexpr int T = 64 * WGM * WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16, F = BN / 4;
@@ -117,7 +117,7 @@ __device__ __forceinline__ bool staged_epilogue(const f4 (&acc)[BM / WGM / 16][B
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   const bool act4 = epi.act == 4, act2 = epi.act == 2;
   // C's columns: 2 N (act 4), N / 2 (act 2), else N; j stays a multiple of 4
-  const bool ok = n0 + BN <= N && (PO || (a16(C) && ldc % 4 == 0)) && (!epi.bias || a16(epi.bias)) &&
+  const bool ok = n0 + BN <= N && a16(C) && ldc % 4 == 0 && (!epi.bias || a16(epi.bias)) &&
                   (!epi.cin || (a16(epi.cin) && epi.ldcin % 4 == 0)) && (!epi.pre || (a16(epi.pre) && epi.ldpre % 4 == 0));
   if (!ok) return false;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
@@ -125,47 +125,13 @@ __device__ __forceinline__ bool staged_epilogue(const f4 (&acc)[BM / WGM / 16][B
   auto slot = [](int R, int q) { return R * BN + 4 * (q ^ ((4 * (R >> 2)) & (F - 1))); };
   const int q = tid % F;
   const int j = n0 + 4 * q;
-  // a thread's NO outputs of row i from output column jo on: to C, or (block
-  // pairs) split by the power of two that puts the largest |output| of the
-  // row's BN-column tile at [2^14, 2^15) -- the row's F threads are
-  // consecutive lanes, F 16 or 32 -- with one thread a row writing the
-  // inverse scale
+  // a thread's NO outputs of row i from output column jo on
   auto put = [&](int i, int jo, const float* o, auto no_c) {
     constexpr int NO = decltype(no_c)::value;
-    if constexpr (!PO) {
-      float* dst = C + int64_t(i) * ldc + jo;
-      if constexpr (NO == 2) *reinterpret_cast<float2*>(dst) = make_float2(o[0], o[1]);
-      if constexpr (NO >= 4) *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-      if constexpr (NO == 8) *reinterpret_cast<float4*>(dst + 4) = make_float4(o[4], o[5], o[6], o[7]);
-    } else {
-    static_assert(F == 16 || F == 32, "a row's threads one or two DPP rows");
-    float m = 0.f;
-#pragma unroll
-    for (int e = 0; e < NO; ++e) m = fmaxf(m, fabsf(o[e]));
-    int mb = __float_as_int(m);  // |values|: the bit patterns order as the values
-#define PET_ROR(n) mb = max(mb, __builtin_amdgcn_update_dpp(0, mb, 0x120 + (n), 0xf, 0xf, true))
-    PET_ROR(1);
-    PET_ROR(2);
-    PET_ROR(4);
-    PET_ROR(8);
-#undef PET_ROR
-    if constexpr (F == 32) mb = max(mb, __shfl_xor(mb, 16));
-    const float sc = pair_scale(__int_as_float(mb));
-    unsigned h[NO / 2], lw[NO / 2];
-#pragma unroll
-    for (int e = 0; e < NO / 2; ++e) pair2(o[2 * e] * sc, o[2 * e + 1] * sc, h[e], lw[e]);
-    unsigned* hi = reinterpret_cast<unsigned*>(epi.pout + (int64_t(i) * epi.kgo + jo / 8) * 2) + (jo % 8) / 2;
-    if constexpr (NO == 2) hi[0] = h[0], hi[4] = lw[0];
-    if constexpr (NO == 4) {
-      *reinterpret_cast<u2*>(hi) = u2{h[0], h[1]};
-      *reinterpret_cast<u2*>(hi + 4) = u2{lw[0], lw[1]};
-    }
-    if constexpr (NO == 8) {
-      *reinterpret_cast<u4*>(hi) = u4{h[0], h[1], h[2], h[3]};
-      *reinterpret_cast<u4*>(hi + 4) = u4{lw[0], lw[1], lw[2], lw[3]};
-    }
-    if (q == 0) epi.pinv[int64_t(n0 / BN) * epi.ldinv + i] = 1.f / sc;
-    }
+    float* dst = C + int64_t(i) * ldc + jo;
+    if constexpr (NO == 2) *reinterpret_cast<float2*>(dst) = make_float2(o[0], o[1]);
+    if constexpr (NO >= 4) *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+    if constexpr (NO == 8) *reinterpret_cast<float4*>(dst + 4) = make_float4(o[4], o[5], o[6], o[7]);
   };
   using c2 = std::integral_constant<int, 2>;
   using c4 = std::integral_constant<int, 4>;
@@ -508,194 +474,6 @@ __global__ void split_rows_kernel(const float* __restrict__ W, int N, int K, int
   for (int p = 0; p < 3; ++p) out[t * 3 + p] = parts[p];
 }
 
-// C = epi(A B^T) with B as fp16 pairs made once (pair_rows_kernel:
-// per row, per 8-element k group, its hi and lo parts, 32 bytes, then the
-// rows' inverse scales) and A split as each k step of 32 is staged, after a
-// first pass over the tile's rows for their scales. Tiles of WGM x WGN waves
-// (64 WGM WGN threads): 64 x 64 or 128 x 64 of 2 x 2, 128 x 128 of 2 x 4. K
-// steps of 32 go through one LDS buffer, the next step's slices loaded into
-// registers under the current step's products. A row's step is 4 groups x 2
-// parts x 16 bytes plus a 16-byte pad (9 u4: 16 consecutive rows' 128-bit
-// operand reads fall on distinct banks). K a multiple of 32.
-//
-// BF: B comes as fp32 rows [N, K] (ld ldb) and is split as it is staged, like
-// A (for a caller with no room to keep a split copy), its row scales from the
-// same first pass.
-template <int BM, int BN, int WGM = 2, int WGN = 2, bool BF = false>
-__global__ void __launch_bounds__(64 * WGM * WGN) __attribute__((amdgpu_waves_per_eu(BN == 128 ? 4 : BM == 128 ? 2 : 3))) gemm_nt_pair_kernel(int M, int N, int K,
-                                                                       const float* __restrict__ A, int64_t lda,
-                                                                       const u4* __restrict__ Bs, float* C,
-                                                                       int64_t ldc, Epi epi,
-                                                                       const float* __restrict__ Bf, int64_t ldb,
-                                                                       int cpw) {
-  constexpr int T = 64 * WGM * WGN, NW = T / 64, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16, RP = 9;
-  constexpr int AL = BM * 8 / T;  // float4 of a step's A slice, a thread's share
-  constexpr int BL = BN * 8 / T;  // B slice: float4 (BF) or u4 slots, a thread's share
-  static_assert(AL * T == BM * 8 && BL * T == BN * 8, "a step's slices divide evenly over the threads");
-  __shared__ u4 lds_ab[(BM + BN) * RP];  // A's and B's step slices, one array (the epilogue's tile spans both)
-  u4* const As = lds_ab;
-  u4* const Bt = lds_ab + BM * RP;
-  __shared__ float sa[BM], sb[BF ? BN : 1];  // row scales of the tile's A rows (and B rows with BF)
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
-  const int wm = w / WGN, wn = w % WGN;
-  // Workgroups go to the 8 XCDs in turn (an L2 each): XCD k takes a
-  // contiguous run of tiles in row-block order, so a row block's column tiles
-  // share an L2 (509730 x 512 x 512: 1547 against 1624 us in launch order).
-  // A bijection of the tiles whatever the hardware's order.
-  // A 1-D grid of work items, item t = (row block t / NG, its column tiles
-  // cpw (t % NG) .. in turn): the A rows' scales are found once for cpw tiles.
-  const int NT = (N + BN - 1) / BN, NG = (NT + cpw - 1) / cpw, total = gridDim.x, L = blockIdx.x;
-  const int q = total / 8, r = total % 8, x = L % 8;
-  const int t = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + L / 8;
-  const int tm = t / NG, tn0 = (t % NG) * cpw, tn1 = min(tn0 + cpw, NT);
-  const int m0 = tm * BM, KG = K / 8;
-  int n0 = tn0 * BN;
-
-  // The first pass: wave w takes rows w, w + NW, ..., a float4 a lane along
-  // k, all its rows' loads in flight together, then each row's largest |x|
-  // reduced over the wave. Rows past M (N) read the last row: their results
-  // are never stored.
-  auto row_scales = [&](const float* X, int64_t ldx, int rows, auto nr, float* s) {
-    constexpr int RW = decltype(nr)::value / NW, RB = RW < 8 ? RW : 8;  // rows a wave, a batch
-#pragma unroll
-    for (int j0 = 0; j0 < RW; j0 += RB) {
-      unsigned o[RB];  // row offsets from X (a tile's rows: within 2^32 floats)
-      float m[RB];
-#pragma unroll
-      for (int j = 0; j < RB; ++j) o[j] = unsigned(min(w + NW * (j0 + j), rows - 1)) * unsigned(ldx), m[j] = 0.f;
-      for (int k = 4 * l; k < K; k += 256) {
-        float4 v[RB];
-#pragma unroll
-        for (int j = 0; j < RB; ++j) v[j] = *reinterpret_cast<const float4*>(X + o[j] + k);
-#pragma unroll
-        for (int j = 0; j < RB; ++j)
-          m[j] = fmaxf(m[j], fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
-      }
-#pragma unroll
-      for (int j = 0; j < RB; ++j) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], o));
-        if (l == 0) s[w + NW * (j0 + j)] = pair_scale(m[j]);
-      }
-    }
-  };
-  row_scales(A + int64_t(m0) * lda, lda, M - m0, std::integral_constant<int, BM>(), sa);
-  __syncthreads();
-
-  // A: thread t's float4 slots q = t + T u, row q / 8, k 4 (q % 8) .. ;
-  // B: u4 slots q, row q / 8, part (q % 8) of the row's step
-  float4 ra[AL];
-  float rsa[AL];
-  u4 rb[BF ? 1 : BL];
-  float4 rbf[BF ? BL : 1];
-  float rsb[BF ? BL : 1];
-  const float* pa[AL];
-#pragma unroll
-  for (int u = 0; u < AL; ++u) {
-    const int qq = tid + T * u;
-    pa[u] = A + int64_t(min(m0 + qq / 8, M - 1)) * lda + 4 * (qq % 8);
-    rsa[u] = sa[qq / 8];
-  }
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < AL; ++u) ra[u] = *reinterpret_cast<const float4*>(pa[u] + k0);
-#pragma unroll
-    for (int u = 0; u < BL; ++u) {
-      const int qq = tid + T * u, j = min(n0 + qq / 8, N - 1);
-      if constexpr (BF)
-        rbf[u] = *reinterpret_cast<const float4*>(Bf + int64_t(j) * ldb + k0 + 4 * (qq % 8));
-      else
-        rb[u] = Bs[(int64_t(j) * KG + k0 / 8) * 2 + qq % 8];
-    }
-  };
-  // a float4 of row `row`'s k slots 4 (q % 8) .. , scaled by s, into its
-  // row's hi and lo parts of k group (q % 8) / 2, half q & 1, of tile X
-  auto store_pair = [&](u4* X, int row, int qq, const float4& v, float s) {
-    unsigned h0, l0, h1, l1;
-    pair2(v.x * s, v.y * s, h0, l0);
-    pair2(v.z * s, v.w * s, h1, l1);
-    unsigned* dst = reinterpret_cast<unsigned*>(&X[row * RP + ((qq % 8) / 2) * 2]) + 2 * (qq & 1);
-    *reinterpret_cast<uint2*>(dst) = make_uint2(h0, h1);
-    *reinterpret_cast<uint2*>(dst + 4) = make_uint2(l0, l1);
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int u = 0; u < AL; ++u) {
-      const int qq = tid + T * u;
-      store_pair(As, qq / 8, qq, ra[u], rsa[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < BL; ++u) {
-      const int qq = tid + T * u;
-      if constexpr (BF)
-        store_pair(Bt, qq / 8, qq, rbf[u], rsb[u]);
-      else
-        Bt[(qq / 8) * RP + qq % 8] = rb[u];
-    }
-  };
-
-  const int steps = K / 32;
-  for (int tn = tn0; tn < tn1; ++tn) {
-  n0 = tn * BN;
-  if constexpr (BF) {
-    row_scales(Bf + int64_t(n0) * ldb, ldb, N - n0, std::integral_constant<int, BN>(), sb);
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < BL; ++u) rsb[u] = sb[(tid + T * u) / 8];
-  }
-  f4 acc[TM][TN];
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-  load(0);
-  store();
-  __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    if (s + 1 < steps) load((s + 1) * 32);
-    u4 av[TM][2], bv[TN][2];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) av[a][p] = As[(wm * WM + 16 * a + c) * RP + 2 * g + p];
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) bv[b][p] = Bt[(wn * WN + 16 * b + c) * RP + 2 * g + p];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int b = 0; b < TN; ++b) acc[a][b] = mfma3(av[a], bv[b], acc[a][b]);
-    if (s + 1 < steps) {
-      __syncthreads();  // every wave is done with the step's slices
-      store();
-      __syncthreads();
-    }
-  }
-  // the scales undone: rows 4g + r of each 16-row block (from LDS), this
-  // lane's columns (from the split weights' inverse scales, or LDS with BF)
-  const float* inv_b = reinterpret_cast<const float*>(Bs + int64_t(N) * KG * 2);
-#pragma unroll
-  for (int b = 0; b < TN; ++b) {
-    const int jj = wn * WN + 16 * b + c;
-    const float ib = BF ? 1.f / sb[jj] : inv_b[min(n0 + jj, N - 1)];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) acc[a][b][rr] = acc[a][b][rr] * (1.f / sa[wm * WM + 16 * a + 4 * g + rr]) * ib;
-  }
-  // (m0 laundered per tile: the epilogue's row addresses are then made
-  // here, not hoisted out of the tile loop into registers held across it)
-  int m0t = m0;
-  asm volatile("" : "+s"(m0t));
-  // through LDS (As and Bt, done with), a pass per wave row
-  static_assert((BM / WGM) * BN * 4 <= (BM + BN) * RP * 16, "a wave row's results fit the slices' LDS");
-  if (!staged_epilogue<BM, BN, WGM, WGN, WGM>(acc, reinterpret_cast<float*>(As), m0t, n0, M, N, C, ldc, epi))
-    epilogue<WM, WN>(acc, m0t, n0, wm, wn, c, g, M, N, C, ldc, epi);
-  __syncthreads();  // the next tile's first slices overwrite this one's last
-  }
-}
-
 // Rows of B = W (transposed false: W [N, K], ld ldw) or B = W^T (transposed
 // true: W [K, N]) as P fp16 parts: out[(n K/8 + j) P + p] = part p of row n's
 // k group j, scaled by the row's s_n (P 2: hi and lo, pair2; P 3: hi, mid and
@@ -789,187 +567,6 @@ __global__ void __launch_bounds__(256) pair_act_kernel(const float* __restrict__
   if (l == 0) reinterpret_cast<float*>(out + int64_t(M) * KG * 2)[row] = 1.f / s;
 }
 
-// C = epi(A B^T) with both operands as fp16 pairs (pair_act_kernel's and
-// pair_rows_kernel's layout): a row's K step of 32 is 8 u4, part p = 2 group +
-// (0 hi, 1 lo). No vector arithmetic in the K loop: the steps go from global
-// memory straight into an LDS ring of ST stages (global_load_lds_dwordx4, a
-// wave's instruction filling 8 rows' steps, 1 KB), ST - 1 steps in flight, one
-// barrier a step. Part p of row r sits in 16-byte slot p ^ f(r) of the row's
-// 128 bytes, f(r) = bit 2 of r as bit 0 and bit 3 as bit 2: a 128-bit LDS
-// read serves 32 lanes (16 rows, two k groups) a cycle over 128 banks, rows
-// r, r + 4, r + 8, r + 12 share banks, and f gives their two groups' slots
-// {x, x ^ 2} four disjoint pairs (measured: f = r & 7 2-way conflicts, 17% of
-// cycles; f = (r >> 1) & 7 25%). The swizzle is applied on the global side
-// (lane L of an instruction loads the part its slot L % 8 holds). The k order and the
-// epilogue's unscaling are gemm_nt_pair_kernel's, so the two give the same bits.
-// Tiles of WGM x WGN waves; K a multiple of 32.
-// KBS > 0: A as block pairs (a staged epilogue's pout): A's scale is per (row,
-// K block of 32 KBS), the inverse scales [K / (32 KBS)][M] after the pairs.
-// Each block's products go to their own accumulators (cleared at the block's
-// start), which are then added into the total times the rows'
-// inverse scales for the block (staged in LDS after the ring at the start);
-// B's column scales are undone at the end.
-// PO: the output as block pairs (Epi::pout) from the staged epilogue.
-template <int BM, int BN, int WGM, int WGN, int ST, int KBS = 0, bool PO = false>
-__global__ void __launch_bounds__(64 * WGM * WGN)
-__attribute__((amdgpu_waves_per_eu(BM == 128 && BN == 128 ? 4 : 1))) gemm_pp_kernel(int M, int N, int K, const u4* __restrict__ Ap,
-                                                                  const u4* __restrict__ Bs, float* C, int64_t ldc,
-                                                                  Epi epi, int WR) {
-  constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
-  constexpr int SR = BM + BN, LPW = SR / 8 / NW;  // rows a stage; load instructions a wave a step
-  static_assert(LPW * 8 * NW == SR && ST >= 2 && ST <= 6, "a stage's rows divide over the waves");
-  extern __shared__ u4 ring[];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
-  const int wm = w / WGN, wn = w % WGN;
-  // the XCD-contiguous tile order of gemm_nt_pair_kernel, one tile an item;
-  // within an XCD's run, windows of WR row blocks, each swept column tile by
-  // column tile with its row blocks fastest: the tiles in flight at once are
-  // a few row blocks by a few column tiles, whose A rows and B strip both
-  // stay in the XCD's L2 (row-block order instead streamed all of B, 4 MB at
-  // N 2048, through each row block: 2.6 times the product's bytes)
-  const int NT = (N + BN - 1) / BN, RB = (M + BM - 1) / BM, total = gridDim.x, L = blockIdx.x;
-  const int q = total / 8, r = total % 8, x = L % 8;
-  const int t = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + L / 8;
-  const int wi = t / (WR * NT), wr = min(WR, RB - wi * WR), within = t - wi * WR * NT;
-  const int m0 = (wi * WR + within % wr) * BM, n0 = (within / wr) * BN, KG = K / 8;
-
-  // this lane's source for each of the wave's load instructions: stage row
-  // R = 8 (w LPW + i) + l / 8 (A rows first, then B), part (l % 8) ^ (l / 8)
-  const u4* src[LPW];
-#pragma unroll
-  for (int i = 0; i < LPW; ++i) {
-    const int R = 8 * (w * LPW + i) + (l >> 3), p = (l & 7) ^ (((R >> 2) & 1) | ((R >> 1) & 4));
-    src[i] = R < BM ? Ap + int64_t(min(m0 + R, M - 1)) * KG * 2 + p
-                    : Bs + int64_t(min(n0 + R - BM, N - 1)) * KG * 2 + p;
-  }
-  const int steps = K / 32;
-  auto issue = [&](int s) {
-    u4* dst = ring + (s % ST) * SR * 8 + w * LPW * 64;
-#pragma unroll
-    for (int i = 0; i < LPW; ++i)
-      ring_load(src[i] + 8 * s, dst + 64 * i);
-  };
-  f4 acc[TM][TN];
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-  // block pairs: the tile's rows' inverse scales of every K block into LDS
-  // after the ring (the loads issued before the ring's first steps, the
-  // stores after them)
-  constexpr int SPT = KBS > 0 ? (32 * BM + 64 * NW - 1) / (64 * NW) : 1;  // scales a thread, at most 32 blocks
-  float* scl = reinterpret_cast<float*>(ring + ST * SR * 8);
-  const int nblk = KBS > 0 ? steps / KBS : 0;
-  float sv[SPT];
-  if constexpr (KBS > 0) {
-    const float* inv_a = reinterpret_cast<const float*>(Ap + int64_t(M) * KG * 2);
-#pragma unroll
-    for (int u = 0; u < SPT; ++u) {
-      const int ti = tid + 64 * NW * u, kb = ti / BM, rw = ti % BM;
-      sv[u] = kb < nblk ? inv_a[int64_t(kb) * M + min(m0 + rw, M - 1)] : 0.f;
-    }
-  }
-#pragma unroll
-  for (int s = 0; s < ST - 1; ++s)
-    if (s < steps) issue(s);
-  if constexpr (KBS > 0) {
-#pragma unroll
-    for (int u = 0; u < SPT; ++u) {
-      const int ti = tid + 64 * NW * u;
-      if (ti < nblk * BM) scl[ti] = sv[u];
-    }
-  }
-  const int fc = ((c >> 2) & 1) | ((c >> 1) & 4);  // f(row), row & 15 = c
-  const int sw0 = (2 * g) ^ fc, sw1 = (2 * g + 1) ^ fc;
-  // step s: its loads done (those after it may still fly), every wave's
-  // reads of the stage it refills done, the refill issued, the products
-  auto step = [&](int s) {
-    const int after = min(ST - 2, steps - 1 - s);
-    if (after >= ST - 2) wait_vm<(ST - 2) * LPW>();
-    else if constexpr (ST >= 4) {
-      if (after == 1) wait_vm<LPW>();
-      else if (ST >= 5 && after == 2) wait_vm<2 * LPW>();
-      else if (ST >= 6 && after == 3) wait_vm<3 * LPW>();
-      else wait_vm<0>();
-    } else {
-      wait_vm<0>();
-    }
-    ring_barrier();
-    if (s + ST - 1 < steps) issue(s + ST - 1);  // into the stage step s - 1 used
-    const u4* st = ring + (s % ST) * SR * 8;
-    u4 av[TM][2], bv[TN][2];
-#pragma unroll
-    for (int a = 0; a < TM; ++a) {
-      const u4* row = st + (wm * WM + 16 * a + c) * 8;
-      av[a][0] = row[sw0], av[a][1] = row[sw1];
-    }
-#pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      const u4* row = st + (BM + wn * WN + 16 * b + c) * 8;
-      bv[b][0] = row[sw0], bv[b][1] = row[sw1];
-    }
-    // mfma3's three products (hi lo, lo hi, hi hi), each over every tile
-    // before the next: TM TN independent accumulators between two dependent
-    // instructions, the same sums in the same order
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-          acc[a][b] = pet_split::mfma_h(av[a][p == 0 ? 1 : 0], bv[b][p == 1 ? 1 : 0], acc[a][b]);
-  };
-  const float* inv_b = reinterpret_cast<const float*>(Bs + int64_t(N) * KG * 2);
-  if constexpr (KBS == 0) {
-    for (int s = 0; s < steps; ++s) step(s);
-    const float* inv_a = reinterpret_cast<const float*>(Ap + int64_t(M) * KG * 2);
-#pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      const float ib = inv_b[min(n0 + wn * WN + 16 * b + c, N - 1)];
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr)
-          acc[a][b][rr] = acc[a][b][rr] * inv_a[min(m0 + wm * WM + 16 * a + 4 * g + rr, M - 1)] * ib;
-    }
-  } else {
-    f4 tot[TM][TN];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int b = 0; b < TN; ++b) tot[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int kb = 0; kb < nblk; ++kb) {
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int ss = 0; ss < KBS; ++ss) step(kb * KBS + ss);
-      // the block into the total, times its rows' inverse scales (rows 4g .. 4g + 3 of each tile)
-#pragma unroll
-      for (int a = 0; a < TM; ++a) {
-        const float4 ia = *reinterpret_cast<const float4*>(scl + kb * BM + wm * WM + 16 * a + 4 * g);
-        const float iar[4] = {ia.x, ia.y, ia.z, ia.w};
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) tot[a][b][rr] = fmaf(acc[a][b][rr], iar[rr], tot[a][b][rr]);
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      const float ib = inv_b[min(n0 + wn * WN + 16 * b + c, N - 1)];
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) acc[a][b][rr] = tot[a][b][rr] * ib;
-    }
-  }
-  static_assert(ST * (BM + BN) * 128 >= BM * BN * 4, "the ring holds the result tile");
-  if (staged_epilogue<BM, BN, WGM, WGN, 1, PO>(acc, reinterpret_cast<float*>(ring), m0, n0, M, N, C, ldc, epi)) return;
-  if constexpr (!PO) epilogue<WM, WN>(acc, m0, n0, wm, wn, c, g, M, N, C, ldc, epi);  // (block pairs: the host makes sure of the staged one)
-}
-
 }  // namespace pet_gemm
 
 using namespace pet_gemm;
@@ -1039,19 +636,16 @@ extern "C" int pet_linear_fused(int M, int N, int K, const float* A, int64_t lda
 }
 
 int pet_gemm_nt_pp(int M, int N, int K, const void* Ap, const void* Bs, float* C, int64_t ldc, const Epi& e,
-                   hipStream_t st, bool tile128 = false);
+                   hipStream_t st);
 int pet_gemm_pair_rows(const float* X, int M, int K, int64_t ldx, void* out, hipStream_t st);
 
-// The pairs-by-pairs path's threshold: from N = 512 the products' gain
-// outweighs splitting A (C5 energy+forces on MI355X, same bits: N >= 1024
-// 176.4 ms, N >= 512 171.4, N >= 256 171.4, never 191; plain products, same
-// process: 131072 x 1536 x 512 1060 against 95 + 800 us, 498338 x 2048 x 512
-// 4634 against 342 + 3443; with a kept pre-activation 5760 against 4244).
-constexpr int kPairsMinN = 512;
+// From which N A's rows are split into the scratch first: below, their scales
+// are found by each tile (62291 rows on MI355X: N 512 K 1024 236 us against 75 + 176,
+// N 2048 K 512 519 against 45 + 408; the same bits). Block pairs out ask for the
+// scratch from N = 512.
+constexpr int kPairsMinN = 1024, kBlocksMinN = 512;
 
-// The split-product GEMM with the epilogue e (block pairs out where e.pout:
-// then 128 x 128 tiles, so that an output row's K blocks are 128 columns of
-// the product wide).
+// The split-product GEMM with the epilogue e (block pairs out where e.pout).
 int split_impl(int M, int N, int K, const float* A, int64_t lda, const void* Bs, float* C, int64_t ldc, Epi e,
                hipStream_t st, void* scratch, size_t scratch_bytes) {
   if (M < 0 || N < 0 || K < 0) return PET_ATTN_EINVAL;
@@ -1062,13 +656,12 @@ int split_impl(int M, int N, int K, const float* A, int64_t lda, const void* Bs,
     return PET_ATTN_EALIGN;
   if (e.act == 2 && N % 2) return PET_ATTN_EINVAL;
   const int64_t ldcin = e.ldcin, ldpre = e.ldpre;
-  const bool t128 = e.pout != nullptr;
   // A's rows split into the scratch a chunk at a time (as many rows as it
   // holds, a multiple of 128), each chunk's product from the pairs
   const int64_t chunk = scratch ? int64_t(scratch_bytes / (size_t(K) * 4 + 4)) / 128 * 128 : 0;
-  const bool pp = pair_form(K) && N >= kPairsMinN && chunk >= 128 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0;
-  if (t128 && !pp) return PET_ATTN_EINVAL;  // block pairs out: the pairs-by-pairs kernel only
-  if (pp) {
+  const bool room = pair_form(K) && N >= kBlocksMinN && chunk >= 128 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0;
+  if (e.pout && !room) return PET_ATTN_EINVAL;  // block pairs out: as many rows of scratch as that path has always asked for
+  if (e.pout || (room && N >= kPairsMinN)) {
     for (int64_t r0 = 0; r0 < M; r0 += chunk) {
       const int m = int(std::min<int64_t>(chunk, M - r0));
       Epi ec = e;
@@ -1077,23 +670,17 @@ int split_impl(int M, int N, int K, const float* A, int64_t lda, const void* Bs,
       if (ec.pre) ec.pre += r0 * ldpre;
       if (ec.pout) ec.pout += r0 * ec.kgo * 2, ec.pinv += r0;
       int rc = pet_gemm_pair_rows(A + r0 * lda, m, K, lda, scratch, st);
-      if (rc == PET_ATTN_OK) rc = pet_gemm_nt_pp(m, N, K, scratch, Bs, C ? C + r0 * ldc : C, ldc, ec, st, t128);
+      if (rc == PET_ATTN_OK) rc = pet_gemm_nt_pp(m, N, K, scratch, Bs, C ? C + r0 * ldc : C, ldc, ec, st);
       if (rc != PET_ATTN_OK) return rc;
     }
     return PET_ATTN_OK;
   }
-  auto go = [&](auto kern, int bm, int bn, int threads, bool pair) {  // a 1-D grid of every work item
-    const int64_t rb = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-    // column tiles per item (pair kernel): about 2048 items, four rounds of
-    // two workgroups a CU (the rows' scales are found once an item; measured
-    // against 1024, 1536 and 3072 items: 131072 x 1536 x 512 842 against
-    // 883-850 us, 131072 x 512 x 2048 1062 against 1203-1055 us)
-    const int64_t c0 = pair ? std::max<int64_t>(1, std::min<int64_t>(nt, rb * nt / 2048)) : 1;
-    const int64_t ng = (nt + c0 - 1) / c0, cpw = (nt + ng - 1) / ng;
-    hipLaunchKernelGGL(kern, dim3(unsigned(rb * ((nt + cpw - 1) / cpw))), dim3(threads), 0, st, M, N, K, A, lda,
-                       static_cast<const u4*>(Bs), C, ldc, e, static_cast<const float*>(nullptr), int64_t(0),
-                       int(cpw));
-    tally(pair ? 2 : 1, M, N, K);
+  if (pair_form(K)) return pet_gemm_nt_rows(M, N, K, A, lda, kRowsExact, 0, Bs, 2, C, ldc, e, st, 0);
+  auto go = [&](auto kern, int bm, int bn, int threads) {  // a 1-D grid of every tile
+    const int64_t tiles = int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    hipLaunchKernelGGL(kern, dim3(unsigned(tiles)), dim3(threads), 0, st, M, N, K, A, lda, static_cast<const u4*>(Bs), C,
+                       ldc, e, static_cast<const float*>(nullptr), int64_t(0), 1);
+    tally(1, M, N, K);
   };
   // measured on MI355X: 128 x 128 tiles of 8 waves where there are many
   // (131072 x 1536 x 512: 1200-1213 us against 1394-1418 for 128 x 64 and
@@ -1101,21 +688,12 @@ int split_impl(int M, int N, int K, const float* A, int64_t lda, const void* Bs,
   // faster), 64 x 64 otherwise (27318 x 128 x 128: 16.1 against 18.4 us); one
   // LDS buffer beat two in every shape
   const int64_t tiles128 = int64_t((M + 127) / 128) * ((N + 63) / 64);
-  if (pair_form(K)) {
-    if (t128 || (N >= 128 && tiles128 >= 2048))
-      go(gemm_nt_pair_kernel<128, 128, 2, 4>, 128, 128, 512, true);
-    else if (tiles128 >= 2048)
-      go(gemm_nt_pair_kernel<128, 64>, 128, 64, 256, true);
-    else
-      go(gemm_nt_pair_kernel<64, 64>, 64, 64, 256, true);
-  } else {
-    if (t128 || (N >= 128 && tiles128 >= 2048))
-      go(gemm_nt_split_kernel<128, 128, 2, 4>, 128, 128, 512, false);
-    else if (tiles128 >= 2048)
-      go(gemm_nt_split_kernel<128, 64>, 128, 64, 256, false);
-    else
-      go(gemm_nt_split_kernel<64, 64>, 64, 64, 256, false);
-  }
+  if (N >= 128 && tiles128 >= 2048)
+    go(gemm_nt_split_kernel<128, 128, 2, 4>, 128, 128, 512);
+  else if (tiles128 >= 2048)
+    go(gemm_nt_split_kernel<128, 64>, 128, 64, 256);
+  else
+    go(gemm_nt_split_kernel<64, 64>, 64, 64, 256);
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
 }
 
@@ -1261,64 +839,13 @@ int pet_gemm_pair_rows(const float* X, int M, int K, int64_t ldx, void* out, hip
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
 }
 
-// The pairs-by-pairs kernel's shapes: tile, waves, LDS stages.
-struct PPShape {
-  void (*kern)(int, int, int, const u4*, const u4*, float*, int64_t, Epi, int);
-  int bm, bn, threads, stages;
-  size_t lds() const { return size_t(stages) * (bm + bn) * 128; }
-};
-// measured on MI355X (131072 x 1536 x 512, plain epilogue): 128 x 128 tiles
-// of 8 waves with two stages (two workgroups a CU) 752-813 us; four stages (one
-// workgroup) 1128; three 991; 256 x 128 tiles, three stages 827-874; 128 x
-// 128 of 4 waves 1300; the operand reads of the next step issued before this
-// step's products (a second register set, three or four stages) 695-1018
-const PPShape kPP[] = {
-    {gemm_pp_kernel<128, 128, 2, 4, 2>, 128, 128, 512, 2},  // many tiles, N >= 128
-    {gemm_pp_kernel<128, 64, 2, 2, 4>, 128, 64, 256, 4},    // fewer tiles, N >= 64
-    {gemm_pp_kernel<64, 64, 2, 2, 4>, 64, 64, 256, 4},      // the rest
-};
-// the first shape with block pairs out (Epi::pout)
-const PPShape kPPOut = {gemm_pp_kernel<128, 128, 2, 4, 2, 0, true>, 128, 128, 512, 2};
-
 // C = epi(A B^T) from the pairs of A (pet_gemm_pair_rows) and of B
 // (pet_gemm_split_weights), K of the pair form.
 int pet_gemm_nt_pp(int M, int N, int K, const void* Ap, const void* Bs, float* C, int64_t ldc, const Epi& e,
-                   hipStream_t st, bool tile128) {
+                   hipStream_t st) {
   if (M < 0 || N < 0 || !pair_form(K) || K % 32) return PET_ATTN_EINVAL;
   if (M == 0 || N == 0) return PET_ATTN_OK;
-  if ((reinterpret_cast<uintptr_t>(Ap) & 15) || (reinterpret_cast<uintptr_t>(Bs) & 15)) return PET_ATTN_EALIGN;
-  if (int64_t((M + 63) / 64) * ((N + 63) / 64) >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
-  // each shape's dynamic LDS above the 64 KB default, set once a device (the
-  // attribute is the current device's) for every shape
-  static std::mutex mu;
-  static signed char set_on[64] = {};  // 0 not yet, 1 set, -1 failed
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return PET_ATTN_ELAUNCH;
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    if (set_on[dev] == 0) {
-      set_on[dev] = 1;
-      for (const PPShape& k : kPP)
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(k.kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                int(k.lds())) != hipSuccess)
-          set_on[dev] = -1;
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kPPOut.kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              int(kPPOut.lds())) != hipSuccess)
-        set_on[dev] = -1;
-    }
-    if (set_on[dev] < 0) return PET_ATTN_ELAUNCH;
-  }
-  const int64_t t128 = int64_t((M + 127) / 128) * ((N + 127) / 128);
-  const PPShape& k = e.pout ? kPPOut : kPP[tile128 || (N >= 128 && t128 >= 1024) ? 0 : N >= 64 ? 1 : 2];
-  const int64_t tiles = int64_t((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
-  // windows of 8 row blocks (498338 x 2048 x 512 on MI355X: L2-miss reads
-  // 4.55 -> 2.71 GiB a product, 3587 -> 3428 us; 16 the same time, 2 and 4
-  // between)
-  constexpr int wr = 8;
-  hipLaunchKernelGGL(k.kern, dim3(unsigned(tiles)), dim3(k.threads), k.lds(), st, M, N, K,
-                     static_cast<const u4*>(Ap), static_cast<const u4*>(Bs), C, ldc, e, wr);
-  tally(2, M, N, K);
-  return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
+  return pet_gemm_nt_rows(M, N, K, Ap, 0, kRowsPairs, K, Bs, 2, C, ldc, e, st, 0);
 }
 
 // Block pairs out (as pet_gemm_nt_split_pairs) from A already as pair rows
@@ -1337,31 +864,10 @@ int pet_gemm_nt_pp_to_blocks(int M, int N, int K, const void* Ap, const void* Bs
   e.pout = static_cast<u4*>(pout), e.kgo = no / 8, e.ldinv = M;
   e.pinv = reinterpret_cast<float*>(e.pout + int64_t(M) * e.kgo * 2);
   if (kb) *kb = out_cols(128, act);
-  return pet_gemm_nt_pp(M, N, K, Ap, Bs, nullptr, 0, e, st, true);
+  return pet_gemm_nt_pp(M, N, K, Ap, Bs, nullptr, 0, e, st);
 }
 
-// The block-pairs product's kernels: kPP's shapes, by K block of 32, 64, 128
-// or 256 (KBS 1, 2, 4, 8 steps); each takes at most 32 blocks' scales in LDS
-// after its ring.
-using PPKern = void (*)(int, int, int, const u4*, const u4*, float*, int64_t, Epi, int);
 constexpr int kMaxBlocks = 32;
-PPKern pp_blocks_kernel(int shape, int kbs) {
-  switch (shape * 16 + kbs) {
-    case 1: return gemm_pp_kernel<128, 128, 2, 4, 2, 1>;
-    case 2: return gemm_pp_kernel<128, 128, 2, 4, 2, 2>;
-    case 4: return gemm_pp_kernel<128, 128, 2, 4, 2, 4>;
-    case 8: return gemm_pp_kernel<128, 128, 2, 4, 2, 8>;
-    case 17: return gemm_pp_kernel<128, 64, 2, 2, 4, 1>;
-    case 18: return gemm_pp_kernel<128, 64, 2, 2, 4, 2>;
-    case 20: return gemm_pp_kernel<128, 64, 2, 2, 4, 4>;
-    case 24: return gemm_pp_kernel<128, 64, 2, 2, 4, 8>;
-    case 33: return gemm_pp_kernel<64, 64, 2, 2, 4, 1>;
-    case 34: return gemm_pp_kernel<64, 64, 2, 2, 4, 2>;
-    case 36: return gemm_pp_kernel<64, 64, 2, 2, 4, 4>;
-    case 40: return gemm_pp_kernel<64, 64, 2, 2, 4, 8>;
-    default: return nullptr;
-  }
-}
 
 // C = epi(A B^T) with A as block pairs (pet_gemm_nt_split_pairs' pout: M
 // rows of pairs, then the inverse scales [K / kb][M]) and B's pair rows; kb 32,
@@ -1373,37 +879,10 @@ int pet_gemm_nt_pp_blocks(int M, int N, int K, const void* Ap, int kb, const voi
       K / kb > kMaxBlocks || (act == 2 && N % 2))
     return PET_ATTN_EINVAL;
   if (M == 0 || N == 0) return PET_ATTN_OK;
-  if ((reinterpret_cast<uintptr_t>(Ap) & 15) || (reinterpret_cast<uintptr_t>(Bs) & 15)) return PET_ATTN_EALIGN;
-  if (int64_t((M + 63) / 64) * ((N + 63) / 64) >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
-  static std::mutex mu;
-  static signed char set_on[64] = {};  // 0 not yet, 1 set, -1 failed
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return PET_ATTN_ELAUNCH;
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    if (set_on[dev] == 0) {
-      set_on[dev] = 1;
-      for (int sh = 0; sh < 3; ++sh)
-        for (int kbs : {1, 2, 4, 8})
-          if (hipFuncSetAttribute(reinterpret_cast<const void*>(pp_blocks_kernel(sh, kbs)),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  int(kPP[sh].lds() + size_t(kMaxBlocks) * kPP[sh].bm * 4)) != hipSuccess)
-            set_on[dev] = -1;
-    }
-    if (set_on[dev] < 0) return PET_ATTN_ELAUNCH;
-  }
   Epi e;
   e.row_scale = row_scale, e.bias = bias, e.cin = cin, e.ldcin = ldcin, e.beta = beta, e.pre = pre, e.ldpre = ldpre;
   e.act = act;
-  const int64_t t128 = int64_t((M + 127) / 128) * ((N + 127) / 128);
-  const int sh = N >= 128 && t128 >= 1024 ? 0 : N >= 64 ? 1 : 2;
-  const PPShape& k = kPP[sh];
-  const int64_t tiles = int64_t((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
-  const size_t lds = k.lds() + size_t(K / kb) * k.bm * 4;
-  hipLaunchKernelGGL(pp_blocks_kernel(sh, kb / 32), dim3(unsigned(tiles)), dim3(k.threads), lds, st, M, N, K,
-                     static_cast<const u4*>(Ap), static_cast<const u4*>(Bs), C, ldc, e, 8);
-  tally(2, M, N, K);
-  return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
+  return pet_gemm_nt_rows(M, N, K, Ap, 0, kRowsPairs, kb, Bs, 2, C, ldc, e, st, 0);
 }
 
 // B's rows as three fp16 parts (hi, mid, lo: W exactly) at any K (a multiple

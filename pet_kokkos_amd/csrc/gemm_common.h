@@ -32,7 +32,7 @@ struct Epi {
   int64_t ldpre = 0;
   int act = 0;                       // 0 none, 1 SiLU, 2 SwiGLU (C has N/2 columns),
                                      // 3 / 4 the backward of SiLU / SwiGLU (below)
-  // Block pairs in place of C (staged epilogue only): the output row i as
+  // Block pairs in place of C (the row kernels only): the output row i as
   // fp16 pairs in pair_act_kernel's layout (kgo k groups of 8 a row, each
   // group's hi then lo 16 bytes), scaled per (row, column tile) -- the tile's
   // output columns are one K block of the product that reads them -- with the
@@ -209,3 +209,7 @@ __device__ __forceinline__ void wait_vm() {
 // gemm_rows.hip: C = epilogue(A B^T) from three-part weights (pet_gemm_pair_weights)
 int pet_gemm_nt_p3(int M, int N, int K, const float* A, int64_t lda, const void* Bp, float* C, int64_t ldc,
                    const pet_gemm::Epi& e, hipStream_t st);
+// ... and on the row kernels, P parts of weights a value; as: how A comes
+enum { kRowsOnline = 0, kRowsExact = 1, kRowsPairs = 2 };
+int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, int kb, const void* Bp, int P, float* C,
+                     int64_t ldc, const pet_gemm::Epi& e, hipStream_t st, int cfg);

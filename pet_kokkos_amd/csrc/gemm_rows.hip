@@ -50,8 +50,8 @@ namespace pet_gemm {
 using pet_attn::max_g;
 using pet_split::mfma_h;
 
-enum { kOnline = 0, kExact = 1, kPairs = 2 };    // A
-enum { kVec = 0, kAny = 1, kBlocks = 2 };        // the output: fp32 with 16-byte accesses, any fp32, block pairs
+enum { kOnline = kRowsOnline, kExact = kRowsExact, kPairs = kRowsPairs };  // A
+enum { kVec = 0, kAny = 1, kBlocks = 2 };  // the output: fp32 with 16-byte accesses, any fp32, block pairs
 
 namespace {
 
@@ -102,8 +102,8 @@ __device__ __forceinline__ float outgrow(float m, float& sa, float& lim) {
   return f;
 }
 
-// Three-part products sum each step of 32 from zero and add the step to the
-// running sum, the rows of odd steps negated and their sums subtracted. The
+// A step of 32 is summed from zero and added to the running sum; with three-part
+// weights the rows of odd steps are negated and their sums subtracted. The
 // matrix instruction rounds its sums, and each product as it aligns it, toward
 // minus infinity: summed in place, an error of 1.6e-7 (K 128) to 3.2e-7 (K 512) of
 // a result with a mean of -1.6e-8 to -3.3e-8 that a model sums over its atoms
@@ -335,7 +335,11 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
   }
 }
 
-// ACT classes of an epilogue: 0 none or SiLU, 2 SwiGLU, 3 / 4 the backwards.
+// The tile kernel. From pairs it takes the place of a kernel with 128 x 128 tiles
+// of eight waves that read 12 operand fragments for 24 instructions a step and met
+// LDS bank conflicts (MI355X, 62291 rows: 512 x 2048 424 -> 337 us, 512 x 1024 237 -> 176,
+// 2048 x 512 424 -> 408); from fp32 rows, of one that split them on their way into LDS
+// (26670 x 128 x 1024: 58.5 -> 48.6).
 template <int TM, int TN, int WR, int WC, int P, int AS, int OUT>
 __global__ void __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(rows_waves(TM, TN))))
 gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, float* C, int64_t ldc, Epi epi, int kbs,
@@ -434,7 +438,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
 #pragma unroll
   for (int s = 0; s < ST - 1; ++s) issue(s, s);
 
-  f4 ts[P == 3 ? NG > 1 ? 2 : 1 : 1][TM][TG];  // a group's step
+  f4 ts[NG > 1 ? 2 : 1][TM][TG];  // a group's step
   auto add_group = [&](auto set, int bg) {
     constexpr int X = decltype(set)::value;
 #pragma unroll
@@ -481,10 +485,8 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
     read(c0_{}, 0);
     if constexpr (NG > 1) read(c1_{}, 1);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (P == 3) {
-      if (s) add_group(last_{}, NG - 1);
-      sg = s & 1 ? -1.f : 1.f;
-    }
+    if (s) add_group(last_{}, NG - 1);
+    if constexpr (P == 3) sg = s & 1 ? -1.f : 1.f;
     if constexpr (AS == kPairs) {
       if (kbs < steps) {
         if (left == 0) {  // a block begins: its factor, and the next one's scale on its way
@@ -532,26 +534,22 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
     // ones; a group's step is added under the next group's products
     auto products = [&](auto set, int bg) {
       constexpr int X = decltype(set)::value;
-      if constexpr (P == 3)
 #pragma unroll
-        for (int j = 0; j < TG; ++j)
+      for (int j = 0; j < TG; ++j)
 #pragma unroll
-          for (int a = 0; a < TM; ++a) ts[X][a][j] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int a = 0; a < TM; ++a) ts[X][a][j] = f4{0.f, 0.f, 0.f, 0.f};
       auto prod = [&](int p, const u4* a_) {
 #pragma unroll
         for (int j = 0; j < TG; ++j)
 #pragma unroll
-          for (int a = 0; a < TM; ++a) {
-            f4& d = P == 3 ? ts[X][a][j] : acc[a][TG * bg + j];
-            d = mfma_h(wv[X][j][p], a_[a], d);
-          }
+          for (int a = 0; a < TM; ++a) ts[X][a][j] = mfma_h(wv[X][j][p], a_[a], ts[X][a][j]);
       };
       if constexpr (P == 2) {
         prod(0, al), prod(1, ah), prod(0, ah);
       } else {
         prod(1, al), prod(2, ah), prod(0, al), prod(1, ah), prod(0, ah);
-        if (bg > 0) add_group(std::integral_constant<int, X ^ 1>{}, bg - 1);
       }
+      if (bg > 0) add_group(std::integral_constant<int, X ^ 1>{}, bg - 1);
     };
 #pragma unroll
     for (int bg = 0; bg < NG; bg += 2) {
@@ -566,7 +564,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
     }
     stage = stage + 1 == ST ? 0 : stage + 1;
   }
-  if constexpr (P == 3) add_group(last_{}, NG - 1);
+  add_group(last_{}, NG - 1);
   wait_vm<0>();  // no load into LDS outlives the loop
 
   // ---- epilogue
@@ -897,8 +895,7 @@ RowsShape rows_pick(int cfg) {
 // from K = 256: 2; pet_gemm_pair_weights: 3); as: how A comes (kOnline,
 // kExact: fp32 rows, 16-byte aligned; kPairs: pair rows or blocks of kb
 // columns). K a multiple of 32; e.pout: block pairs in place of C (N a multiple
-// of 128, every operand 16-byte aligned). cfg: a shape to force, for tests and
-// measurement (0: chosen).
+// of 128, A as pairs, every operand 16-byte aligned). cfg: the shape (0: chosen here).
 int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, int kb, const void* Bp, int P, float* C,
                      int64_t ldc, const Epi& e, hipStream_t st, int cfg) {
   if (M < 0 || N < 0 || K < 32 || K % 32 || (as == kPairs && (kb < 32 || kb % 32 || K % kb))) return PET_ATTN_EINVAL;
@@ -911,23 +908,30 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
   auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(64, 32) >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
   if (!cfg) {
+    // 256 x 256 tiles (one workgroup a CU) where their last round of 256 leaves
+    // at most a sixth of the CUs idle over all rounds: full, they are 1.13 to 1.17 times
+    // faster than 128 x 128 (62291 x 512 x 1024 from pairs: 176 against 204 us, 488
+    // tiles; 26670 x 1024 x 512 with SwiGLU: 102 against 94, 420 tiles). An
+    // activation's backward into block pairs is bound by its operand: 128 x 128
+    // there (62291 x 1024 x 512, SwiGLU: 324 against 382).
+    const int64_t t256 = tiles(256, 256), rounds = (t256 + 255) / 256;
+    const bool c1 = N > 128 && 6 * t256 >= 5 * 256 * rounds;
     if (e.pout)
-      cfg = tiles(256, 256) >= 256 && N % 256 == 0 ? 1 : 6;
+      cfg = c1 && N % 256 == 0 && e.act <= 2 ? 1 : 6;
     else
-      cfg = P == 2 && N > 128 && tiles(256, 256) >= 512 ? 1 : N > 64 && tiles(128, 128) >= 512 ? 2 : N > 64 && tiles(64, 128) >= 512 ? 3 : N > 32 && tiles(64, 64) >= 256 ? 4 : 5;
+      cfg = P == 2 && c1 ? 1 : N > 64 && tiles(128, 128) >= 512 ? 2 : N > 64 && tiles(64, 128) > 256 ? 3 : tiles(64, 64) >= 256 ? 4 : 5;
   }
   RowsShape s;
   using std::integral_constant;
   auto pick = [&](auto p, auto a) {
     constexpr int P_ = decltype(p)::value, A_ = decltype(a)::value;
     if (e.pout) {
-      if constexpr (P_ == 2) s = rows_pick<P_, A_, kBlocks>(cfg);
+      if constexpr (P_ == 2 && A_ == kPairs) s = rows_pick<P_, A_, kBlocks>(cfg);
     } else {
       s = vec ? rows_pick<P_, A_, kVec>(cfg) : rows_pick<P_, A_, kAny>(cfg);
     }
   };
   if (P == 3 && as == kOnline) pick(integral_constant<int, 3>{}, integral_constant<int, kOnline>{});
-  else if (P == 2 && as == kOnline) pick(integral_constant<int, 2>{}, integral_constant<int, kOnline>{});
   else if (P == 2 && as == kExact) pick(integral_constant<int, 2>{}, integral_constant<int, kExact>{});
   else if (P == 2 && as == kPairs) pick(integral_constant<int, 2>{}, integral_constant<int, kPairs>{});
   if (!s.k) return PET_ATTN_EINVAL;

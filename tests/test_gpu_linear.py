@@ -646,3 +646,45 @@ def test_three_part_kernels(M, N, K, device):
         L.fused(A[lo:hi].clone(), P, H2, bias=b, pre=pre2, act=2)
         assert torch.equal(H[lo:hi], H2) and torch.equal(pre[lo:hi], pre2)
         assert ((pre.double() - z).abs() <= tol).all()
+
+
+# 256 x 256 tiles (27419 rows) and 128 x 128 or smaller (999) for both products
+@pytest.mark.parametrize("M", [999, 27419])
+@pytest.mark.parametrize("act", [1, 2])
+def test_block_pairs_unlike_blocks(M, act, device):
+    """Blocks of one row far apart (2^-30, 1 and 2^20, and a block of zeros, and a
+    row of zeros) out of one product and into the next, which brings a row's
+    blocks to its smallest scale: an element's error within the sums' rounding
+    (2^-20 of sum |x| |w| as the short-K kernels', one more bit for the weights'
+    pairs) and 2^-38 of the row's largest |x| times sum |w| for the bits a small
+    block loses below the row's fp16 subnormals."""
+    N0, K0, N = 512, 256, 384
+    g = torch.Generator(device=device).manual_seed(M + act)
+    A = torch.randn(M, K0, device=device, generator=g)
+    A[5] = 0
+    W0 = torch.randn(N0, K0, device=device, generator=g) / K0 ** 0.5
+    W0[128:256] = 0
+    gate = torch.zeros(N0, dtype=torch.bool, device=device)
+    gate[1::2] = act == 2
+    scale = torch.ones(N0, device=device)
+    scale[256:384], scale[384:] = 2.0 ** -30, 2.0 ** 20
+    W0 = torch.where(gate[:, None], W0, W0 * scale[:, None])
+    scratch = torch.empty(M * (K0 + 1) + 64, device=device)
+    cols = N0 // 2 if act == 2 else N0
+    B = L.BlockPairs(M, cols, device)
+    L.fused_to_blocks(A, L.SplitWeights(W0), B, act=act, scratch=scratch)
+    x, _ = blocks_ref(B, device)
+    C0 = torch.empty(M, cols, device=device)
+    L.fused(A, L.SplitWeights(W0), C0, act=act)
+    blockmax = C0.double().abs().reshape(M, -1, B.kb).amax(2).repeat_interleave(B.kb, 1)
+    assert ((x - C0.double()).abs() <= 2.0 ** -21 * C0.double().abs() + 2.0 ** -38 * blockmax).all()
+    if act == 1:
+        assert (x[:, 128:256] == 0).all()
+    W = L.SplitWeights(torch.randn(N, cols, device=device, generator=g) / cols ** 0.5)
+    C = torch.full((M, N), float("nan"), device=device)
+    L.fused(B, W, C)
+    w = W_ref(W, device)
+    err = (C.double() - x @ w.T).abs()
+    tol = 2.0 ** -19 * (x.abs() @ w.abs().T) + 2.0 ** -38 * x.abs().amax(1, keepdim=True) * w.abs().sum(1)
+    assert (err <= tol).all()
+    assert (C[5] == 0).all()
