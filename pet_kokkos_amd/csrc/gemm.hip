@@ -886,7 +886,7 @@ int pet_gemm_nt_pp_blocks(int M, int N, int K, const void* Ap, int kb, const voi
 }
 
 // B's rows as three fp16 parts (hi, mid, lo: W exactly) at any K (a multiple
-// of 32), for the short-K kernel: N K 6 + N 4 bytes.
+// of 32), for the three-part kernels: N K 6 + N 4 bytes.
 int pet_gemm_pair_weights(const float* W, int N, int K, int64_t ldw, bool transposed, void* out, hipStream_t st) {
   if (N < 0 || K < 0 || K % 32 || (reinterpret_cast<uintptr_t>(out) & 15)) return PET_ATTN_EINVAL;
   if (N == 0 || K == 0) return PET_ATTN_OK;

@@ -46,7 +46,7 @@ struct Epi {
 // FLOPs (2 M N K) of the products this library's dense kernels have launched,
 // by the instructions that run them: 0 the fp32 fused kernel (fp32 matrix
 // cores), 1 split-fp32 as three bf16 parts (six bf16 products), 2 fp16 pairs
-// (three fp16 products), 3 the short-K kernel (five fp16 products). A
+// (three fp16 products), 3 the three-part kernels (five fp16 products). A
 // measurement aid, process-wide (pet_gemm_flop_tally).
 extern std::atomic<uint64_t> g_flops[4];  // gemm.hip
 inline void tally(int cls, int64_t M, int64_t N, int64_t K) {
