@@ -247,6 +247,17 @@ def test_attention_layer_fwd_bwd(device, ln, dead, cfg):
     assert rel(csa.cpu().numpy(), rcsa) <= RTOL
 
 
+@pytest.mark.parametrize("ln", [False, True])
+@pytest.mark.parametrize("dead", [False, True])
+def test_attention_layer_three_part_products(device, ln, dead):
+    """The same chain at C2's layer (27 thousand rows of width 128): its products
+    lie between 2^27 and 2^32, on the three-part kernels, the weights' split
+    copies following one another in one piece of the workspace."""
+    conf, tk = systems.config_tokens("c2")
+    assert 2 ** 27 <= tk.n_rows * conf.d_model ** 2 and 3 * tk.n_rows * conf.d_model ** 2 < 2 ** 32
+    test_attention_layer_fwd_bwd(device, ln, dead, "c2")
+
+
 def test_layer_to_forces_chain(device):
     """The path end to end on C1: the layer's backward accumulates cf_seq_adj,
     which the edge term turns into per-edge gradients and the fold into forces,
