@@ -208,8 +208,8 @@ PET_ATTN_API int pet_linear_fused_pairs(int M, int N, int K, const void* Apairs,
  * for SwiGLU, 256 for its backward, 128 otherwise). Every epilogue operand
  * 16-byte aligned, leading dimensions multiples of 4.
  * pet_linear_fused_blocks is pet_linear_fused_pairs with A as such blocks (K =
- * out_cols, kb as returned, at most 32 blocks): each block's products summed
- * on their own, then into the total times the block's inverse scale. No
+ * out_cols, kb as returned, at most 32 blocks): each step of 32 summed on its
+ * own, then into the total at the row's smallest block scale. No
  * counterpart in the reference, whose fused layers (src/fused_gemm_hip.cpp:345-400)
  * write fp32. */
 PET_ATTN_API int pet_linear_fused_split_blocks(int M, int N, int K, const float* A, int64_t lda, const void* Wsplit,

@@ -27,9 +27,10 @@
 //   kExact: the row's largest |x| is found first, in a pass over the wave's rows
 //     (whose second reading comes from cache): the bits of the pair rows
 //     (pair_act_kernel) read in form kPairs.
-//   kPairs: A already as fp16 pairs with a scale per (row, K block): the row's
-//     blocks are brought to the row's smallest scale by a power of two as they
-//     are read (exact, but for bits 2^-39 below the row's largest).
+//   kPairs: A already as fp16 pairs with a scale per (row, K block): a step's
+//     sum, made from zero at its block's own scale, is brought to the row's
+//     smallest scale in fp32 as it is added, so that a block far below the row's
+//     largest keeps all of its bits.
 // A row's results depend on that row alone, and repeat bit for bit.
 #include <hip/hip_runtime.h>
 
@@ -78,10 +79,6 @@ __device__ __forceinline__ void split8x(u4& x, u4& y, float s) {
     x[j] = __builtin_bit_cast(unsigned, h);
     y[j] = __builtin_bit_cast(unsigned, lo);
   }
-}
-
-__device__ __forceinline__ unsigned h2_mul(unsigned x, unsigned f) {
-  return __builtin_bit_cast(unsigned, pet_split::h2v(__builtin_bit_cast(pet_split::h2v, x) * __builtin_bit_cast(pet_split::h2v, f)));
 }
 
 // A row's running scale sa (kOnline) once |x| up to m, this lane's share of the
@@ -396,9 +393,12 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
     for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
   // the row's scale and the largest |x| it takes (kOnline), 1 / scale at the end
   float sa[TM], lim[TM], sg = 1.f;
-  // kPairs: the row's largest inverse scale, the current block's factor onto it
-  float imax[TM], inext[TM];
-  unsigned fac[TM];
+  // kPairs: the row's largest inverse scale (as its exponent field, a byte a row:
+  // registers), the current block's factor onto it (a power of two, at most 1:
+  // the fp16 operands themselves would lose bits to it, or with a factor below
+  // 2^-24 the whole block)
+  unsigned imax = 0;
+  float inext[TM], fac[TM];
   const float* inv_a = nullptr;
   float* smax = reinterpret_cast<float*>(lds + ST * Sh::STAGE);
   if constexpr (AS == kExact) {
@@ -430,9 +430,9 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
       const int row = min(m0 + 16 * a + c, M - 1);
       float m = 0.f;
       for (int b = g; b < nblk; b += 4) m = fmaxf(m, inv_a[int64_t(b) * M + row]);
-      imax[a] = max_g(m);
+      imax |= (__float_as_uint(max_g(m)) >> 23) << (8 * a);
       inext[a] = inv_a[row];
-      fac[a] = 0x3c003c00u;  // 1, 1
+      fac[a] = 1.f;
     }
   }
 #pragma unroll
@@ -444,7 +444,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
 #pragma unroll
     for (int j = 0; j < TG; ++j)
 #pragma unroll
-      for (int a = 0; a < TM; ++a) add_step(acc[a][TG * bg + j], ts[X][a][j], sg);
+      for (int a = 0; a < TM; ++a) add_step(acc[a][TG * bg + j], ts[X][a][j], AS == kPairs ? fac[a] : sg);
   };
   using last_ = std::integral_constant<int, (NG > 1 ? 1 : 0)>;  // the last group's set
   int stage = 0;          // step s's
@@ -493,17 +493,11 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
           left = kbs, blk = min(blk + 1, steps / kbs - 1);
 #pragma unroll
           for (int a = 0; a < TM; ++a) {
-            const float f = __builtin_amdgcn_ldexpf(inext[a], 1 - __builtin_amdgcn_frexp_expf(imax[a]));
-            const pet_split::h2v f2 = {(_Float16)f, (_Float16)f};
-            fac[a] = __builtin_bit_cast(unsigned, f2);
+            fac[a] = inext[a] * __uint_as_float((254 - (imax >> (8 * a) & 255)) << 23);
             inext[a] = inv_a[int64_t(blk) * M + min(m0 + 16 * a + c, M - 1)];
           }
         }
         --left;
-#pragma unroll
-        for (int a = 0; a < TM; ++a)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) ah[a][j] = h2_mul(ah[a][j], fac[a]), al[a][j] = h2_mul(al[a][j], fac[a]);
       }
     } else {
       if constexpr (AS == kExact) {
@@ -570,7 +564,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   // ---- epilogue
   float ia[TM];
 #pragma unroll
-  for (int a = 0; a < TM; ++a) ia[a] = AS == kPairs ? imax[a] : 1.f / sa[a];
+  for (int a = 0; a < TM; ++a) ia[a] = AS == kPairs ? __uint_as_float((imax >> (8 * a) & 255) << 23) : 1.f / sa[a];
   rows_epilogue<TM, TN, OUT>(acc, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0, n0, c, g, M, N, C,
                              ldc, epi);
 }

@@ -653,11 +653,10 @@ def test_three_part_kernels(M, N, K, device):
 @pytest.mark.parametrize("act", [1, 2])
 def test_block_pairs_unlike_blocks(M, act, device):
     """Blocks of one row far apart (2^-30, 1 and 2^20, and a block of zeros, and a
-    row of zeros) out of one product and into the next, which brings a row's
-    blocks to its smallest scale: an element's error within the sums' rounding
-    (2^-20 of sum |x| |w| as the short-K kernels', one more bit for the weights'
-    pairs) and 2^-38 of the row's largest |x| times sum |w| for the bits a small
-    block loses below the row's fp16 subnormals."""
+    row of zeros) out of one product and into the next, which brings each
+    step's sum to the row's smallest scale: an element's error within the sums'
+    rounding (2^-20 of sum |x| |w| as the three-part kernels', one more bit for
+    the weights' pairs)."""
     N0, K0, N = 512, 256, 384
     g = torch.Generator(device=device).manual_seed(M + act)
     A = torch.randn(M, K0, device=device, generator=g)
@@ -685,6 +684,32 @@ def test_block_pairs_unlike_blocks(M, act, device):
     L.fused(B, W, C)
     w = W_ref(W, device)
     err = (C.double() - x @ w.T).abs()
-    tol = 2.0 ** -19 * (x.abs() @ w.abs().T) + 2.0 ** -38 * x.abs().amax(1, keepdim=True) * w.abs().sum(1)
-    assert (err <= tol).all()
+    assert (err <= 2.0 ** -19 * (x.abs() @ w.abs().T)).all()
     assert (C[5] == 0).all()
+
+
+# 256 x 256 tiles, 128 x 128 or smaller ones; block pairs out of the second too
+@pytest.mark.parametrize("M", [999, 27419])
+@pytest.mark.parametrize("apart", [20, 24, 26, 30, 36, 60, 100])
+def test_block_pairs_small_blocks_kept(M, apart, device):
+    """A row's blocks 2^apart apart, and output columns whose weights are zero
+    on the large block: their sums hold the small blocks alone, with the same
+    relative error as any other (2^-19 of sum |x| |w|, test_block_pairs_unlike_blocks)."""
+    N0, K0, N = 512, 256, 384
+    g = torch.Generator(device=device).manual_seed(M + apart)
+    A = torch.randn(M, K0, device=device, generator=g)
+    W0 = torch.randn(N0, K0, device=device, generator=g) / K0 ** 0.5
+    W0[:128] *= 2.0 ** apart  # the first block of every row
+    W0[256:384] *= 2.0 ** -7
+    B = L.BlockPairs(M, N0, device)
+    L.fused_to_blocks(A, L.SplitWeights(W0), B, scratch=torch.empty(M * (K0 + 1) + 64, device=device))
+    x, _ = blocks_ref(B, device)
+    Wf = torch.randn(N, N0, device=device, generator=g) / N0 ** 0.5
+    Wf[N // 2:, :128] = 0
+    W = L.SplitWeights(Wf)
+    C = torch.full((M, N), float("nan"), device=device)
+    L.fused(B, W, C)
+    w = W_ref(W, device)
+    bound = 2.0 ** -19 * (x.abs() @ w.abs().T)
+    assert (C[:, N // 2:] != 0).all()
+    assert ((C.double() - x @ w.T).abs() <= bound).all()
