@@ -52,7 +52,7 @@ using pet_attn::max_g;
 using pet_split::mfma_h;
 
 enum { kOnline = kRowsOnline, kExact = kRowsExact, kPairs = kRowsPairs };  // A
-enum { kVec = 0, kAny = 1, kBlocks = 2 };  // the output: fp32 with 16-byte accesses, any fp32, block pairs
+enum { kVec = 0, kAny = 1, kBlocks = 2 };  // the output: fp32 of a width a multiple of 4, of any width, block pairs
 
 namespace {
 
@@ -161,6 +161,41 @@ __device__ __forceinline__ void quad_transpose(float (&x)[4]) {
   x[0] = b1 ? u2 : y0, x[1] = b1 ? u3 : y1, x[2] = b1 ? y2 : u0, x[3] = b1 ? y3 : u1;
 }
 
+// n consecutive columns of an epilogue operand. Every address is a float's: the
+// 4-byte alignment of the vectors costs nothing on gfx950 (an access of 16 bytes
+// at any of them is one instruction). Element by element, outputs that are not
+// 16-byte aligned took 1.3 to 2.7 times as long (100000 x 128 x 128 on MI355X: 72 us
+// against 30), and in 256 x 256 tiles, their accumulators in scratch, 12 times
+// (62291 x 512 x 1024 from pairs: 2240 against 181). ANY (the width no multiple of
+// 4): the last chunk's `left` columns one by one.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+template <bool ANY, int n>
+__device__ __forceinline__ void get_cols(const float* p, float (&x)[n], int left) {
+  if (!ANY || left >= n) {
+#pragma unroll
+    for (int e = 0; e < n; e += 4) {
+      const f4u q = *reinterpret_cast<const f4u*>(p + e);
+      x[e] = q[0], x[e + 1] = q[1], x[e + 2] = q[2], x[e + 3] = q[3];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < n; ++e) x[e] = p[min(e, left - 1)];
+  }
+}
+template <bool ANY, int n>
+__device__ __forceinline__ void put_cols(float* p, const float (&x)[n], int left) {
+  if (!ANY || left >= n) {
+    if constexpr (n == 2) *reinterpret_cast<f2u*>(p) = f2u{x[0], x[1]};
+#pragma unroll
+    for (int e = 0; e + 4 <= n; e += 4) *reinterpret_cast<f4u*>(p + e) = f4u{x[e], x[e + 1], x[e + 2], x[e + 3]};
+  } else {
+#pragma unroll
+    for (int e = 0; e < n; ++e)
+      if (e < left) p[e] = x[e];
+  }
+}
+
 }  // namespace
 
 // The epilogue of a wave's TM x TN tiles: acc times the row's inverse scale ia
@@ -176,160 +211,125 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
                                               int m0, int n0, int c, int g, int M, int N, float* C, int64_t ldc,
                                               const Epi& epi) {
   static_assert(TN % 4 == 0, "64 columns at a time");
+  constexpr bool ANY = OUT == kAny;
   const int r0 = m0 + (c & 12), j0 = n0 + 16 * g + 4 * (c & 3);  // this lane's first row and column
-  if constexpr (OUT == kAny) {
+  auto run = [&](auto act) {
+    constexpr int ACT = decltype(act)::value, NG = TN / 4;
+    constexpr int Z = ACT == 4 ? 8 : 4, R = ACT == 2 ? 2 : ACT == 4 ? 8 : 4;  // values read and written a chunk
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+    for (int a = 0; a < TM; ++a) {
+      float res[OUT == kBlocks ? NG : 1][4][R], mx[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int b = 0; b < TN; b += 4) {
+      for (int b = 0; b < NG; ++b) {
+        // (a lane past the last column reads the last ones and writes nothing)
+        const int j = min(j0 + 64 * b, ANY ? N - 1 : N - 4), left = N - j;
+        const bool in = OUT == kBlocks || j0 + 64 * b < N;
+        constexpr int ZC = ACT == 4 ? 2 : 1;  // cin's and the bias's columns a column
+        // the chunk's operands, four rows' together
+        float z[4][Z], ib[4], bb[Z];
+        const bool hz = ACT >= 3 || epi.cin != nullptr;
+        if (hz)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            get_cols<ANY>(epi.cin + int64_t(min(r0 + 16 * a + r, M - 1)) * epi.ldcin + ZC * j, z[r], ZC * left);
+          }
+        get_cols<ANY>(inv_b + j, ib, left);
+        if (epi.bias) get_cols<ANY>(epi.bias + ZC * j, bb, ZC * left);
         float v[4][4];  // [element][row]
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) v[e][s] = acc[a][b + s][e] * ia[a];
+          for (int s = 0; s < 4; ++s) v[e][s] = acc[a][4 * b + s][e] * ia[a];
           quad_transpose(v[e]);
         }
-        const int j = j0 + 16 * b;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float o[4];
+          const int i = r0 + 16 * a + r;
+          const bool live = in && i < M;
+          float u[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = v[e][r] * inv_b[min(j + e, N - 1)];
-          if (epi.act >= 3)
-            epi_quad<false, true>(o, r0 + 16 * a + r, j, M, N, C, ldc, epi);
-          else
-            epi_quad<false, false>(o, r0 + 16 * a + r, j, M, N, C, ldc, epi);
+          for (int e = 0; e < 4; ++e) u[e] = v[e][r] * ib[e];
+          float (&o)[R] = res[OUT == kBlocks ? b : 0][r];
+          if constexpr (ACT == 3) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float x = z[r][e] + (epi.bias ? bb[e] : 0.f), sg = sig_fast(x);
+              o[e] = u[e] * (sg * (1.0f + x * (1.0f - sg)));
+            }
+          } else if constexpr (ACT == 4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float y = z[r][2 * e] + (epi.bias ? bb[2 * e] : 0.f);
+              const float sg = sig_fast(z[r][2 * e + 1] + (epi.bias ? bb[2 * e + 1] : 0.f));
+              o[2 * e] = u[e] * sg, o[2 * e + 1] = u[e] * y * sg * (1.0f - sg);
+            }
+          } else {
+            if (epi.row_scale) {
+              const float rs = epi.row_scale[min(i, M - 1)];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) u[e] *= rs;
+            }
+            if (epi.bias)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) u[e] += bb[e];
+            if (epi.cin)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) u[e] += epi.beta * z[r][e];
+            if (epi.pre && live) put_cols<ANY>(epi.pre + int64_t(i) * epi.ldpre + j, u, left);
+            if constexpr (ACT == 2) {
+              o[0] = u[0] * sig_fast(u[1]), o[1] = u[2] * sig_fast(u[3]);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[e] = epi.act == 1 ? u[e] * sig_fast(u[e]) : u[e];
+            }
+          }
+          if constexpr (OUT != kBlocks) {
+            if (live) put_cols<ANY>(C + int64_t(i) * ldc + (ACT == 2 ? j / 2 : ZC * j), o, ACT == 2 ? left / 2 : ZC * left);
+          } else {
+#pragma unroll
+            for (int e = 0; e < R; ++e) mx[r] = fmaxf(mx[r], fabsf(o[e]));
+          }
+        }
+        if constexpr (OUT != kBlocks) asm volatile("" ::: "memory");  // (the next chunk's operands are not held as well)
+      }
+      if constexpr (OUT == kBlocks) {
+        // each row's 128 columns of the product scaled by their own power of
+        // two, as fp16 pairs: groups of 8 outputs hi then lo, 16 bytes each
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          int m = __float_as_int(mx[r]);  // |values|: the bit patterns order as the values
+          m = max(m, __builtin_amdgcn_update_dpp(0, m, 0xb1, 0xf, 0xf, true));
+          m = max(m, __builtin_amdgcn_update_dpp(0, m, 0x4e, 0xf, 0xf, true));
+          const float sc = pet_split::block_scale(max_g(__int_as_float(m)));
+          const int i = r0 + 16 * a + r;
+          if (i < M) {
+            unsigned* rowp = reinterpret_cast<unsigned*>(epi.pout + int64_t(i) * epi.kgo * 2);
+#pragma unroll
+            for (int b = 0; b < NG; ++b) {
+              const int jo = (ACT == 2 ? 1 : ACT == 4 ? 4 : 2) * (j0 + 64 * b) / 2;  // the first output
+              unsigned h[R / 2], lw[R / 2];
+#pragma unroll
+              for (int e = 0; e < R / 2; ++e)
+                pet_split::pair2(res[b][r][2 * e] * sc, res[b][r][2 * e + 1] * sc, h[e], lw[e]);
+              unsigned* q = rowp + (jo / 8) * 8 + (jo % 8) / 2;
+              if constexpr (R == 2) q[0] = h[0], q[4] = lw[0];
+              if constexpr (R == 4) *reinterpret_cast<u2*>(q) = u2{h[0], h[1]}, *reinterpret_cast<u2*>(q + 4) = u2{lw[0], lw[1]};
+              if constexpr (R == 8) {
+                *reinterpret_cast<u4*>(q) = u4{h[0], h[1], h[2], h[3]};
+                *reinterpret_cast<u4*>(q + 4) = u4{lw[0], lw[1], lw[2], lw[3]};
+              }
+            }
+            if (g == 0 && (c & 3) == 0) epi.pinv[int64_t(n0 / 128) * epi.ldinv + i] = 1.f / sc;
+          }
         }
         asm volatile("" ::: "memory");
       }
-  } else {
-    auto run = [&](auto act) {
-      constexpr int ACT = decltype(act)::value, NG = TN / 4;
-      constexpr int Z = ACT == 4 ? 8 : 4, R = ACT == 2 ? 2 : ACT == 4 ? 8 : 4;  // values read and written a chunk
-#pragma unroll
-      for (int a = 0; a < TM; ++a) {
-        float res[OUT == kBlocks ? NG : 1][4][R], mx[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int b = 0; b < NG; ++b) {
-          const int j = min(j0 + 64 * b, N - 4);  // (N a multiple of 4 in these forms)
-          const bool in = OUT == kBlocks || j0 + 64 * b < N;
-          // the chunk's operands, four rows' together
-          float z[4][Z], ib[4], bb[Z];
-          const bool hz = ACT >= 3 || epi.cin != nullptr;
-          if (hz)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float* zp = epi.cin + int64_t(min(r0 + 16 * a + r, M - 1)) * epi.ldcin + (ACT == 4 ? 2 * j : j);
-#pragma unroll
-              for (int e = 0; e < Z; e += 4) *reinterpret_cast<float4*>(&z[r][e]) = *reinterpret_cast<const float4*>(zp + e);
-            }
-          *reinterpret_cast<float4*>(ib) = *reinterpret_cast<const float4*>(inv_b + j);
-          if (epi.bias)
-#pragma unroll
-            for (int e = 0; e < Z; e += 4)
-              *reinterpret_cast<float4*>(bb + e) = *reinterpret_cast<const float4*>(epi.bias + (ACT == 4 ? 2 * j : j) + e);
-          float v[4][4];  // [element][row]
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) v[e][s] = acc[a][4 * b + s][e] * ia[a];
-            quad_transpose(v[e]);
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = r0 + 16 * a + r;
-            const bool live = in && i < M;
-            float u[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) u[e] = v[e][r] * ib[e];
-            float (&o)[R] = res[OUT == kBlocks ? b : 0][r];
-            if constexpr (ACT == 3) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float x = z[r][e] + (epi.bias ? bb[e] : 0.f), sg = sig_fast(x);
-                o[e] = u[e] * (sg * (1.0f + x * (1.0f - sg)));
-              }
-            } else if constexpr (ACT == 4) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float y = z[r][2 * e] + (epi.bias ? bb[2 * e] : 0.f);
-                const float sg = sig_fast(z[r][2 * e + 1] + (epi.bias ? bb[2 * e + 1] : 0.f));
-                o[2 * e] = u[e] * sg, o[2 * e + 1] = u[e] * y * sg * (1.0f - sg);
-              }
-            } else {
-              if (epi.row_scale) {
-                const float rs = epi.row_scale[min(i, M - 1)];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) u[e] *= rs;
-              }
-              if (epi.bias)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) u[e] += bb[e];
-              if (epi.cin)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) u[e] += epi.beta * z[r][e];
-              if (epi.pre && live)
-                *reinterpret_cast<float4*>(epi.pre + int64_t(i) * epi.ldpre + j) = make_float4(u[0], u[1], u[2], u[3]);
-              if constexpr (ACT == 2) {
-                o[0] = u[0] * sig_fast(u[1]), o[1] = u[2] * sig_fast(u[3]);
-              } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = epi.act == 1 ? u[e] * sig_fast(u[e]) : u[e];
-              }
-            }
-            if constexpr (OUT == kVec) {
-              if (live) {
-                float* cr = C + int64_t(i) * ldc + (ACT == 2 ? j / 2 : ACT == 4 ? 2 * j : j);
-                if constexpr (R == 2) *reinterpret_cast<float2*>(cr) = make_float2(o[0], o[1]);
-#pragma unroll
-                for (int e = 0; e + 4 <= R; e += 4) *reinterpret_cast<float4*>(cr + e) = make_float4(o[e], o[e + 1], o[e + 2], o[e + 3]);
-              }
-            } else {
-#pragma unroll
-              for (int e = 0; e < R; ++e) mx[r] = fmaxf(mx[r], fabsf(o[e]));
-            }
-          }
-          if constexpr (OUT == kVec) asm volatile("" ::: "memory");  // (the next chunk's operands are not held as well)
-        }
-        if constexpr (OUT == kBlocks) {
-          // each row's 128 columns of the product scaled by their own power of
-          // two, as fp16 pairs: groups of 8 outputs hi then lo, 16 bytes each
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            int m = __float_as_int(mx[r]);  // |values|: the bit patterns order as the values
-            m = max(m, __builtin_amdgcn_update_dpp(0, m, 0xb1, 0xf, 0xf, true));
-            m = max(m, __builtin_amdgcn_update_dpp(0, m, 0x4e, 0xf, 0xf, true));
-            const float sc = pet_split::block_scale(max_g(__int_as_float(m)));
-            const int i = r0 + 16 * a + r;
-            if (i < M) {
-              unsigned* rowp = reinterpret_cast<unsigned*>(epi.pout + int64_t(i) * epi.kgo * 2);
-#pragma unroll
-              for (int b = 0; b < NG; ++b) {
-                const int jo = (ACT == 2 ? 1 : ACT == 4 ? 4 : 2) * (j0 + 64 * b) / 2;  // the first output
-                unsigned h[R / 2], lw[R / 2];
-#pragma unroll
-                for (int e = 0; e < R / 2; ++e)
-                  pet_split::pair2(res[b][r][2 * e] * sc, res[b][r][2 * e + 1] * sc, h[e], lw[e]);
-                unsigned* q = rowp + (jo / 8) * 8 + (jo % 8) / 2;
-                if constexpr (R == 2) q[0] = h[0], q[4] = lw[0];
-                if constexpr (R == 4) *reinterpret_cast<u2*>(q) = u2{h[0], h[1]}, *reinterpret_cast<u2*>(q + 4) = u2{lw[0], lw[1]};
-                if constexpr (R == 8) {
-                  *reinterpret_cast<u4*>(q) = u4{h[0], h[1], h[2], h[3]};
-                  *reinterpret_cast<u4*>(q + 4) = u4{lw[0], lw[1], lw[2], lw[3]};
-                }
-              }
-              if (g == 0 && (c & 3) == 0) epi.pinv[int64_t(n0 / 128) * epi.ldinv + i] = 1.f / sc;
-            }
-          }
-          asm volatile("" ::: "memory");
-        }
-      }
-    };
-    if (epi.act == 2) run(std::integral_constant<int, 2>{});
-    else if (epi.act == 3) run(std::integral_constant<int, 3>{});
-    else if (epi.act == 4) run(std::integral_constant<int, 4>{});
-    else run(std::integral_constant<int, 0>{});
-  }
+    }
+  };
+  if (epi.act == 2) run(std::integral_constant<int, 2>{});
+  else if (epi.act == 3) run(std::integral_constant<int, 3>{});
+  else if (epi.act == 4) run(std::integral_constant<int, 4>{});
+  else run(std::integral_constant<int, 0>{});
 }
 
 // The tile kernel. From pairs it takes the place of a kernel with 128 x 128 tiles
@@ -698,7 +698,7 @@ gemm_ksplit_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B,
 // may stand between them. One workgroup a CU (96 KB of weights, 64 KB of
 // slices at K = 128). XCD x takes rows [x M / 8, (x + 1) M / 8), its
 // workgroups S a strip, so the strips re-read A from their L2.
-template <int KB, int TN>
+template <int KB, int TN, int OUT>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_strip_kernel(int M, int N, const float* A, int64_t lda, const u4* B, float* C, int64_t ldc, Epi epi, int S) {
   constexpr int BN = 16 * TN, CH = 12, KG = 4 * KB, NW = 8;
@@ -815,7 +815,7 @@ gemm_strip_kernel(int M, int N, const float* A, int64_t lda, const u4* B, float*
     }
     add_group(std::integral_constant<int, (G - 1) & 1>{}, G - 1);
     const float ia[1] = {1.f / sa};
-    rows_epilogue<1, TN, kVec>(acc, ia, inv_b, xr0 + 16 * blk, n0, c, g, xr1, N, C, ldc, epi);
+    rows_epilogue<1, TN, OUT>(acc, ia, inv_b, xr0 + 16 * blk, n0, c, g, xr1, N, C, ldc, epi);
     // the next block's loads done: issued before the epilogue, whose last
     // stores (four at least: a run's results are one store or more) may still
     // be on their way
@@ -870,7 +870,7 @@ RowsShape rows_pick(int cfg) {
     if (cfg == 1) return rows_shape<4, 8, 4, 2, P, AS, OUT>();
     return rows_shape<2, 8, 4, 1, P, AS, OUT>();
   } else {
-    if constexpr (P == 2)
+    if constexpr (P == 2 && OUT == kVec)
       if (cfg == 1) return rows_shape<4, 8, 4, 2, P, AS, OUT>();
     if (cfg <= 2) return rows_shape<4, 4, 2, 2, P, AS, OUT>();
     if (cfg == 3) return rows_shape<2, 4, 2, 2, P, AS, OUT>();
@@ -897,8 +897,7 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   if ((as != kPairs && lda % 4) || !a16(A) || !a16(Bp)) return PET_ATTN_EALIGN;
   if (e.act == 2 && N % 2) return PET_ATTN_EINVAL;
-  const bool vec = N % 4 == 0 && a16(C) && ldc % 4 == 0 && (!e.bias || a16(e.bias)) &&
-                   (!e.cin || (a16(e.cin) && e.ldcin % 4 == 0)) && (!e.pre || (a16(e.pre) && e.ldpre % 4 == 0));
+  const bool vec = N % 4 == 0;
   auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(64, 32) >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
   if (!cfg) {
@@ -907,9 +906,11 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
     // faster than 128 x 128 (62291 x 512 x 1024 from pairs: 176 against 204 us, 488
     // tiles; 26670 x 1024 x 512 with SwiGLU: 102 against 94, 420 tiles). An
     // activation's backward into block pairs is bound by its operand: 128 x 128
-    // there (62291 x 1024 x 512, SwiGLU: 324 against 382).
+    // there (62291 x 1024 x 512, SwiGLU: 324 against 382). A width that is no
+    // multiple of 4 keeps to 128 x 128: with its last columns one by one the
+    // 256 x 256 epilogue does not fit the registers.
     const int64_t t256 = tiles(256, 256), rounds = (t256 + 255) / 256;
-    const bool c1 = N > 128 && 6 * t256 >= 5 * 256 * rounds;
+    const bool c1 = vec && N > 128 && 6 * t256 >= 5 * 256 * rounds;
     if (e.pout)
       cfg = c1 && N % 256 == 0 && e.act <= 2 ? 1 : 6;
     else
@@ -947,26 +948,26 @@ int pet_gemm_nt_strip(int M, int N, int K, const float* A, int64_t lda, const vo
   auto a16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   if (lda % 4 || !a16(A) || !a16(Bp)) return PET_ATTN_EALIGN;
   if (e.act == 2 && N % 2) return PET_ATTN_EINVAL;
-  const bool vec = N % 4 == 0 && a16(C) && ldc % 4 == 0 && (!e.bias || a16(e.bias)) &&
-                   (!e.cin || (a16(e.cin) && e.ldcin % 4 == 0)) && (!e.pre || (a16(e.pre) && e.ldpre % 4 == 0));
-  if (!vec) return pet_gemm_nt_rows(M, N, K, A, lda, kOnline, 0, Bp, 3, C, ldc, e, st, M < 16384 ? 4 : 3);
   // 64 or 128 columns a workgroup: the strips of an XCD's 32 CUs take
   // ceil(blocks / (8 S)) rounds of 16-row blocks, and a round of 64 columns takes
   // 0.55 of one of 128 (26670 x 512 x 128 with the SwiGLU backward: 44 us with
   // 64, 7 rounds, 51 with 128, 4; 27318 x 128 x 128: 12.4 with 64, 2 rounds,
-  // 11.9 with 128, 1)
+  // 11.9 with 128, 1); a width no multiple of 4 takes 64 (with its last columns one
+  // by one the epilogue of 128 does not fit the registers)
   const int KB = K / 32, nbx = ((M + 7) / 8 + 15) / 16;  // 16-row blocks an XCD
   auto ranges = [&](int bn) {  // row ranges a strip in an XCD
     return std::max(1, std::min(32 / std::min(32, (N + bn - 1) / bn), (nbx + 7) / 8));
   };
   auto rounds = [&](int bn) { return (nbx + 8 * ranges(bn) - 1) / (8 * ranges(bn)); };
-  const int BN = N > 64 && rounds(128) <= 0.55 * rounds(64) ? 128 : 64, NT = (N + BN - 1) / BN, S = ranges(BN);
+  const bool vec = N % 4 == 0;
+  const int BN = vec && N > 64 && rounds(128) <= 0.55 * rounds(64) ? 128 : 64, NT = (N + BN - 1) / BN, S = ranges(BN);
   if (int64_t(8) * NT * S >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
   using K_ = void (*)(int, int, const float*, int64_t, const u4*, float*, int64_t, Epi, int);
   K_ k = nullptr;
   auto pick = [&](auto kb, auto tn) {
     constexpr int KB_ = decltype(kb)::value, TN_ = decltype(tn)::value;
-    k = gemm_strip_kernel<KB_, TN_>;
+    if constexpr (TN_ == 4) k = vec ? gemm_strip_kernel<KB_, 4, kVec> : gemm_strip_kernel<KB_, 4, kAny>;
+    else k = gemm_strip_kernel<KB_, TN_, kVec>;
   };
   auto by_k = [&](auto tn) {
     switch (KB) {
