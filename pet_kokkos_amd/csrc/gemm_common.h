@@ -16,10 +16,11 @@ using pet_split::u2;
 using pet_split::u4;
 
 // The hardware's exp and reciprocal, with one Newton step on the reciprocal
-// (its own ulp of error has a mean that a model's activations add up).
+// (its own ulp of error has a mean that a model's activations add up), except
+// where that is 0 (x below -88): the step would make NaN of it.
 __device__ __forceinline__ float sig_fast(float x) {
-  const float d = fminf(1.0f + __expf(-x), 3.0e38f), r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float d = 1.0f + __expf(-x), r = __builtin_amdgcn_rcpf(d), n = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return r == 0.f ? r : n;
 }
 
 struct Epi {

@@ -135,6 +135,38 @@ def test_backward_epilogues(M, N, K, split, device):
         linear_fused(A, W, C, cin=C, act=5, split=split)
 
 
+@pytest.mark.parametrize("split,K", [(False, 32), (True, 32), (True, 256), ("smallk", 32)],
+                         ids=["fp32", "bf16", "pairs", "smallk"])
+def test_sigmoid_far_out(split, K, device):
+    """The epilogues' sigmoid where exp(-x) passes a float and at NaN: 0 from
+    x = -89 down to -infinity (times any finite value 0), 1 at +infinity, and a
+    NaN stays NaN, in every activation and its backward."""
+    x = torch.tensor([float("nan"), -float("inf"), -3e38, -1e30, -200.0, -90.0, 200.0, float("inf")], device=device)
+    want = torch.tensor([float("nan"), 0, 0, 0, 0, 0, 1, 1], device=device)
+    N, M = 2 * len(x), 5
+    A, W = torch.zeros(M, K, device=device), torch.zeros(N, K, device=device)
+    gates = torch.stack([torch.full_like(x, 2e30), x], 1).reshape(-1)  # (value, gate)
+    H = torch.empty(M, N // 2, device=device)
+    linear_fused(A, W, H, bias=gates, act=2, split=split)
+    assert torch.equal(H.nan_to_num(-7.0), (2e30 * want).expand(M, -1).nan_to_num(-7.0))
+    finite = torch.isfinite(x) | torch.isnan(x)  # (an infinity times a sigmoid of 0 is NaN)
+    z = torch.where(finite, x, torch.zeros_like(x)).repeat(2)
+    C = torch.empty(M, N, device=device)
+    linear_fused(A, W, C, bias=z, act=1, split=split)
+    silu = torch.where(torch.isnan(z), z, z.clamp(min=0)).expand(M, -1)  # 200 there, 0 below
+    assert torch.equal(C.nan_to_num(-7.0).abs(), silu.nan_to_num(-7.0).abs())
+    A[:, 0], W[:, 0] = 1, 3  # an adjoint of 3
+    linear_fused(A, W, C, cin=z.expand(M, -1).contiguous(), act=3, split=split)
+    d = torch.where(z > 0, 3.0, torch.where(z < 0, 0.0, 1.5)) + 0 * torch.where(torch.isnan(z), z, torch.zeros_like(z))
+    assert torch.equal(C.nan_to_num(-7.0).abs(), d.expand(M, -1).nan_to_num(-7.0).abs())
+    C4 = torch.empty(M, 2 * N, device=device)
+    linear_fused(A, W, C4, cin=gates.repeat(2).expand(M, -1).contiguous(), act=4, split=split)
+    g = C4.reshape(M, 2, -1, 2)
+    assert torch.equal(g[..., 0].nan_to_num(-7.0), (3 * want).expand(M, 2, -1).nan_to_num(-7.0))
+    assert torch.equal(torch.isnan(g[..., 1]), torch.isnan(want).expand(M, 2, -1))
+    assert (g[..., 1].nan_to_num(0.0) == 0).all()
+
+
 def test_rejects(device):
     A = torch.zeros(8, 20, device=device)
     W = torch.zeros(8, 20, device=device)
