@@ -174,6 +174,13 @@ PET_ATTN_API int pet_linear_fused_smallk(int M, int N, int K, const float* A, in
                                          float* C, int64_t ldc, const float* row_scale, const float* bias,
                                          const float* cin, int64_t ldcin, float beta, float* pre, int64_t ldpre,
                                          int act, void* stream);
+/* The same at any K a multiple of 32, as the model and the attention layer run
+ * their products below 2^32. Up to K = 224 a row's results depend on that row
+ * alone; from 256 the kernel follows M and N (few rows: the steps are split over
+ * the waves), and a row's last bits with it. */
+PET_ATTN_API int pet_linear_fused_parts(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs, float* C,
+                                        int64_t ldc, const float* row_scale, const float* bias, const float* cin,
+                                        int64_t ldcin, float beta, float* pre, int64_t ldpre, int act, void* stream);
 
 /* Activation rows as fp16 pairs, the A operand of pet_linear_fused_pairs: X [M, K]
  * (ld ldx, K a multiple of 32 and at least 256, rows 16-byte aligned) into out,

@@ -56,6 +56,7 @@ EXPORTS = (
     "pet_linear_pair_weights",
     "pet_attn_access_floor",
     "pet_linear_fused_smallk",
+    "pet_linear_fused_parts",
     "pet_linear_pair_rows",
     "pet_linear_fused_pairs",
     "pet_linear_fused_split_blocks",
@@ -230,8 +231,8 @@ def load() -> ctypes.CDLL:
                                           _P, _P]
     lib.pet_linear_pair_weights.restype = ctypes.c_int
     lib.pet_linear_pair_weights.argtypes = [_P, _I, _I, _I64, _P, _P]
-    lib.pet_linear_fused_smallk.restype = ctypes.c_int
-    lib.pet_linear_fused_smallk.argtypes = [_I, _I, _I, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _F, _P, _I64, _I, _P]
+    lib.pet_linear_fused_smallk.restype = lib.pet_linear_fused_parts.restype = ctypes.c_int
+    lib.pet_linear_fused_smallk.argtypes = lib.pet_linear_fused_parts.argtypes = [_I, _I, _I, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _F, _P, _I64, _I, _P]
     lib.pet_linear_fused_split_ws.restype = ctypes.c_int
     lib.pet_linear_fused_split_ws.argtypes = [_I, _I, _I, _P, _I64, _P, _P, _I64, _P, _P, _P, _I64, _F, _P, _I64, _I,
                                               _P, ctypes.c_size_t, _P]

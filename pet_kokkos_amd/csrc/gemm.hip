@@ -901,9 +901,9 @@ extern "C" int pet_linear_pair_weights(const float* W, int N, int K, int64_t ldw
   return pet_gemm_pair_weights(W, N, K, ldw, false, out, reinterpret_cast<hipStream_t>(stream));
 }
 
-extern "C" int pet_linear_fused_smallk(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs, float* C,
-                                       int64_t ldc, const float* row_scale, const float* bias, const float* cin,
-                                       int64_t ldcin, float beta, float* pre, int64_t ldpre, int act, void* stream) {
+extern "C" int pet_linear_fused_parts(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs, float* C,
+                                      int64_t ldc, const float* row_scale, const float* bias, const float* cin,
+                                      int64_t ldcin, float beta, float* pre, int64_t ldpre, int act, void* stream) {
   if ((M > 0 && N > 0) && (!A || !Wpairs || !C || lda < K || !epi_args_ok(N, C, ldc, row_scale, cin, ldcin, pre,
                                                                               ldpre, act)))
     return PET_ATTN_EINVAL;
@@ -911,8 +911,19 @@ extern "C" int pet_linear_fused_smallk(int M, int N, int K, const float* A, int6
   Epi e;
   e.row_scale = row_scale, e.bias = bias, e.cin = cin, e.ldcin = ldcin, e.beta = beta, e.pre = pre, e.ldpre = ldpre;
   e.act = act;
-  if (K > 128) return PET_ATTN_EINVAL;
   return pet_gemm_nt_p3(M, N, K, A, lda, Wpairs, C, ldc, e, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int pet_linear_fused_smallk(int M, int N, int K, const float* A, int64_t lda, const void* Wpairs, float* C,
+                                       int64_t ldc, const float* row_scale, const float* bias, const float* cin,
+                                       int64_t ldcin, float beta, float* pre, int64_t ldpre, int act, void* stream) {
+  if ((M > 0 && N > 0) && (!A || !Wpairs || !C || lda < K || !epi_args_ok(N, C, ldc, row_scale, cin, ldcin, pre,
+                                                                              ldpre, act)))
+    return PET_ATTN_EINVAL;
+  if (act == 2 && N % 2) return PET_ATTN_EINVAL;
+  if (K > 128) return PET_ATTN_EINVAL;
+  return pet_linear_fused_parts(M, N, K, A, lda, Wpairs, C, ldc, row_scale, bias, cin, ldcin, beta, pre, ldpre, act,
+                                stream);
 }
 
 extern "C" int pet_linear_pair_rows(const float* X, int M, int K, int64_t ldx, void* out, void* stream) {

@@ -39,7 +39,7 @@ class PairWeights:
     """W [N, K] (K a multiple of 32) as rows of three fp16 parts at any K
     (each row scaled by a power of two; hi, mid and lo, their sum W s
     exactly), N K 6 + N 4 bytes: the weights of the short-contraction layer
-    (pet_linear_fused_smallk, K at most 128)."""
+    (pet_linear_fused_smallk, K at most 128) and of fused_parts at any K."""
 
     def __init__(self, W: torch.Tensor):
         _check(W, "W")
@@ -172,7 +172,7 @@ def _check(t, name, rows=None, cols=None, vector=False, device=None):
         raise ValueError(f"{name}: {t.shape[1]} columns, {cols} needed")
 
 
-def _call(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=None, act=0, scratch=None):
+def _call(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=None, act=0, scratch=None, parts=False):
     if act not in (0, 1, 2, 3, 4):
         raise ValueError(f"act {act}: 0 (none), 1 (SiLU), 2 (SwiGLU), 3 / 4 (their backward)")
     if isinstance(A, (PairRows, BlockPairs)):
@@ -215,11 +215,11 @@ def _call(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=None, act=
     st = torch.cuda.current_stream().cuda_stream
     lib = _lib.load()
     if isinstance(W, PairWeights):
-        if isinstance(A, PairRows) or K > 128:
+        if isinstance(A, PairRows) or (K > 128 and not parts):
             raise ValueError("pair weights take fp32 A and K at most 128 (pet_linear_fused_smallk)")
-        _lib.check(lib.pet_linear_fused_smallk(M, N, K, p(A), A.stride(0), W.data.data_ptr(), p(C), C.stride(0),
-                                               p(row_scale), p(bias), p(cin), ld(cin), beta, p(pre), ld(pre), act, st),
-                   "pet_linear_fused_smallk")
+        name = "pet_linear_fused_parts" if parts else "pet_linear_fused_smallk"
+        _lib.check(getattr(lib, name)(M, N, K, p(A), A.stride(0), W.data.data_ptr(), p(C), C.stride(0), p(row_scale),
+                                      p(bias), p(cin), ld(cin), beta, p(pre), ld(pre), act, st), name)
     elif isinstance(A, BlockPairs):
         _lib.check(lib.pet_linear_fused_blocks(M, N, K, A.data.data_ptr(), A.kb, W.data.data_ptr(), p(C), C.stride(0),
                                                p(row_scale), p(bias), p(cin), ld(cin), beta, p(pre), ld(pre), act, st),
@@ -255,6 +255,15 @@ def fused(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=None, act=
     With W as SplitWeights, `scratch` (a device tensor) is the workspace A's
     rows are split into a chunk at a time (pet_linear_fused_split_ws)."""
     _call(A, W, C, row_scale, bias, cin, beta, pre, act, scratch)
+
+
+def fused_parts(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=None, act=0):
+    """fused() with W as PairWeights at any K a multiple of 32
+    (pet_linear_fused_parts), the kernels that the model and the attention
+    layer run below M N K = 2^32."""
+    if not isinstance(W, PairWeights):
+        raise ValueError("fused_parts needs W as PairWeights")
+    _call(A, W, C, row_scale, bias, cin, beta, pre, act, parts=True)
 
 
 def linear_fused(out, inp, W, b=None, beta=0.0):
