@@ -87,14 +87,10 @@ __device__ __forceinline__ void split8x(u4& x, u4& y, float s) {
 __device__ __forceinline__ float outgrow(float m, float& sa, float& lim) {
   const float rm = max_g(m);
   float f = 1.f;
-  if (rm > lim) {
-    if (rm > 3.0e38f) {  // (an infinity: the products are not finite whatever the scale)
-      lim = __builtin_inff();
-    } else {
-      const int k = min(12 - __builtin_amdgcn_frexp_expf(rm), 126);
-      f = __builtin_amdgcn_ldexpf(lim, k - 15);
-      sa = __builtin_amdgcn_ldexpf(1.f, k), lim = __builtin_amdgcn_ldexpf(1.f, 15 - k);
-    }
+  if (rm > lim) {  // (rm finite: infinities are taken out before)
+    const int k = min(12 - __builtin_amdgcn_frexp_expf(rm), 126);
+    f = __builtin_amdgcn_ldexpf(lim, k - 15);
+    sa = __builtin_amdgcn_ldexpf(1.f, k), lim = fminf(__builtin_amdgcn_ldexpf(1.f, 15 - k), pet_split::kFltMax);
   }
   return f;
 }
@@ -161,6 +157,12 @@ __device__ __forceinline__ void quad_transpose(float (&x)[4]) {
   x[0] = b1 ? u2 : y0, x[1] = b1 ? u3 : y1, x[2] = b1 ? y2 : u0, x[3] = b1 ? y3 : u1;
 }
 
+// Lane i of this lane's quad's x.
+template <int i>
+__device__ __forceinline__ int quad_lane(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x55 * i, 0xf, 0xf, true);
+}
+
 // n consecutive columns of an epilogue operand. Every address is a float's: the
 // 4-byte alignment of the vectors costs nothing on gfx950 (an access of 16 bytes
 // at any of them is one instruction). Element by element, outputs that are not
@@ -199,14 +201,18 @@ __device__ __forceinline__ void put_cols(float* p, const float (&x)[n], int left
 }  // namespace
 
 // The epilogue of a wave's TM x TN tiles: acc times the row's inverse scale ia
-// and the columns' inv_b, then epi_elem's arithmetic in its order. A lane holds
+// and the columns' inv_b (a row past 2^64 apart from that factor of its scale,
+// which follows inv_b: sums of 2^30 and more times a scale up to 2^116 can pass the
+// range of a float where the result does not; FAR: three-part weights, whose
+// products ran in fp32, and block pairs out, whose kernel spills 70 registers
+// with it and 101 without), then epi_elem's arithmetic in its order. A lane holds
 // sixteen consecutive columns of its row c; a 4 x 4 transpose of those 16-byte
 // chunks over each quad of lanes makes an instruction's quad cover 64 bytes of
 // one row (r of the four), so a quarter of a wave meets 4 rows' lines, not 16:
 // stores of 16 bytes to 16 rows bounded the products of short K with an
 // activation (26670 x 512 x 128 with SiLU and its kept input on MI355X: 35 us
 // without the transpose, 31 with it).
-template <int TM, int TN, int OUT>
+template <int TM, int TN, int OUT, bool FAR>
 __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const float (&ia)[TM], const float* inv_b,
                                               int m0, int n0, int c, int g, int M, int N, float* C, int64_t ldc,
                                               const Epi& epi) {
@@ -218,6 +224,8 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
     constexpr int Z = ACT == 4 ? 8 : 4, R = ACT == 2 ? 2 : ACT == 4 ? 8 : 4;  // values read and written a chunk
 #pragma unroll
     for (int a = 0; a < TM; ++a) {
+      const bool far = FAR && ia[a] > 0x1p64f, afar = __builtin_amdgcn_ballot_w64(far) != 0;
+      const float ia1 = far ? ia[a] * 0x1p-64f : ia[a];
       float res[OUT == kBlocks ? NG : 1][4][R], mx[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int b = 0; b < NG; ++b) {
@@ -239,7 +247,7 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) v[e][s] = acc[a][4 * b + s][e] * ia[a];
+          for (int s = 0; s < 4; ++s) v[e][s] = acc[a][4 * b + s][e] * ia1;
           quad_transpose(v[e]);
         }
 #pragma unroll
@@ -249,6 +257,12 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
           float u[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) u[e] = v[e][r] * ib[e];
+          if (afar) {
+            const int f = far;
+            const float p = (r == 0 ? quad_lane<0>(f) : r == 1 ? quad_lane<1>(f) : r == 2 ? quad_lane<2>(f) : quad_lane<3>(f)) ? 0x1p64f : 1.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] *= p;
+          }
           float (&o)[R] = res[OUT == kBlocks ? b : 0][r];
           if constexpr (ACT == 3) {
 #pragma unroll
@@ -565,7 +579,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   float ia[TM];
 #pragma unroll
   for (int a = 0; a < TM; ++a) ia[a] = AS == kPairs ? __uint_as_float((imax >> (8 * a) & 255) << 23) : 1.f / sa[a];
-  rows_epilogue<TM, TN, OUT>(acc, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0, n0, c, g, M, N, C,
+  rows_epilogue<TM, TN, OUT, P == 3 || OUT == kBlocks>(acc, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0, n0, c, g, M, N, C,
                              ldc, epi);
 }
 
@@ -583,7 +597,7 @@ gemm_ksplit_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B,
                    int win) {
   constexpr int P = 3, BM = 16 * TM, BN = 16 * TN, CH = 4 * P, LA = BM / 8, LB = BN * CH / 64;
   constexpr int SLICE = BM * 8 + BN * CH;  // 16-byte chunks; the wave's sums (64 TM TN) fit in it
-  static_assert(TN == 4 && TM <= NW && 64 * TM * TN <= SLICE, "the epilogue's 64 columns; a row tile a wave");
+  static_assert(TN == 4 && TM <= NW && 64 * TM * TN + 4 * TM <= SLICE, "the epilogue's 64 columns; a row tile a wave");
   extern __shared__ u4 lds[];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, c = l & 15, g = l >> 4;
   const int KG = K / 8, steps = K / 32;
@@ -667,22 +681,33 @@ gemm_ksplit_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B,
     };
     prod(1, al), prod(2, ah), prod(0, al), prod(1, ah), prod(0, ah);
   }
-  // the waves' sums, each at its rows' own scales, into their slices
+  // the waves' sums and their rows' inverse scales (0: nothing but zeros) into
+  // their slices; a row's sums at the largest of those
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+  for (int a = 0; a < TM; ++a) {
 #pragma unroll
-    for (int b = 0; b < TN; ++b)
-      slice[64 * (a * TN + b) + l] = __builtin_bit_cast(u4, f4(acc[a][b] * (sg / sa[a])));
+    for (int b = 0; b < TN; ++b) slice[64 * (a * TN + b) + l] = __builtin_bit_cast(u4, f4(acc[a][b] * sg));
+    if (g == 0) reinterpret_cast<float*>(slice + 64 * TM * TN)[16 * a + c] = lim[a] > 0.f ? 1.f / sa[a] : 0.f;
+  }
   __syncthreads();
   if (w >= TM) return;
+  float inv[NW], top = 0x1p-126f;
+#pragma unroll
+  for (int v = 0; v < NW; ++v)
+    inv[v] = reinterpret_cast<const float*>(lds + v * SLICE + 64 * TM * TN)[16 * w + c], top = fmaxf(top, inv[v]);
   f4 sum[1][TN];
 #pragma unroll
   for (int b = 0; b < TN; ++b) {
     sum[0][b] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int v = 0; v < min(NW, steps); ++v) sum[0][b] += __builtin_bit_cast(f4, lds[v * SLICE + 64 * (w * TN + b) + l]);
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+      const f4 x = __builtin_bit_cast(f4, lds[v * SLICE + 64 * (w * TN + b) + l]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[0][b][e] = fmaf(x[e], inv[v] * (1.f / top), sum[0][b][e]);
+    }
   }
-  const float one[1] = {1.f};
-  rows_epilogue<1, TN, OUT>(sum, one, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0 + 16 * w, n0, c, g, M,
+  const float ia[1] = {top};
+  rows_epilogue<1, TN, OUT, true>(sum, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0 + 16 * w, n0, c, g, M,
                             N, C, ldc, epi);
 }
 
@@ -815,7 +840,7 @@ gemm_strip_kernel(int M, int N, const float* A, int64_t lda, const u4* B, float*
     }
     add_group(std::integral_constant<int, (G - 1) & 1>{}, G - 1);
     const float ia[1] = {1.f / sa};
-    rows_epilogue<1, TN, OUT>(acc, ia, inv_b, xr0 + 16 * blk, n0, c, g, xr1, N, C, ldc, epi);
+    rows_epilogue<1, TN, OUT, true>(acc, ia, inv_b, xr0 + 16 * blk, n0, c, g, xr1, N, C, ldc, epi);
     // the next block's loads done: issued before the epilogue, whose last
     // stores (four at least: a run's results are one store or more) may still
     // be on their way

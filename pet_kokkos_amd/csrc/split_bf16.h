@@ -115,10 +115,11 @@ __device__ __forceinline__ void pair3(float x, float y, unsigned& hi, unsigned& 
   mid = __builtin_bit_cast(unsigned, m);
   lo = __builtin_bit_cast(unsigned, l);
 }
+constexpr float kFltMax = 3.40282347e38f;
 // The row scale 2^(15 - e) for a largest |x| m = f 2^e (f in [0.5, 1)); 1 for
-// a zero row (and for one holding a NaN, which then propagates).
+// a zero or infinite row (and for one holding a NaN, which then propagates).
 __device__ __forceinline__ float pair_scale(float m) {
-  if (!(m > 0.f) || m > 3.0e38f) return 1.f;
+  if (!(m > 0.f) || m > kFltMax) return 1.f;
   const int e = __builtin_amdgcn_frexp_expf(m);
   return __builtin_amdgcn_ldexpf(1.f, min(15 - e, 126));
 }

@@ -705,6 +705,32 @@ def three_part_kernels(M, N, K, device, alone):
         assert ((pre.double() - z).abs() <= tol).all()
 
 
+# strip, 64 x 64, 32 x 64 tiles; K past 128: 64 x 128, steps split over the waves
+RANGE = [(27011, 128, 128), (27011, 66, 96), (701, 72, 64), (17, 33, 32), (555, 66, 224), (16385, 130, 256),
+         (8191, 128, 1024), (4111, 68, 512), (17, 66, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", RANGE)
+def test_three_part_range(M, N, K, device):
+    """fp32's whole range: rows up to its largest finite value and weights far
+    below and above 1, wherever the result is a normal float. The error is bounded as
+    in three_part_kernels."""
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    ea = torch.tensor([0, 124, -100, 113, 64, -40], device=device)[torch.arange(M, device=device) % 6]
+    ew = torch.tensor([0, -110, 100, -60, 90], device=device)[torch.arange(N, device=device) % 5]
+    A = torch.rand(M, K, device=device, generator=g) - 0.5
+    A = torch.ldexp(A, ea[:, None])
+    A[1::6, K // 3] = torch.finfo(torch.float32).max
+    W = torch.ldexp(torch.rand(N, K, device=device, generator=g) - 0.5, ew[:, None])
+    C = torch.full((M, N), float("nan"), device=device)
+    L.fused_parts(A, L.PairWeights(W), C)
+    ref, mag = A.double() @ W.double().T, A.double().abs() @ W.double().abs().T
+    e = ea[:, None] + ew
+    normal = (e < 110) & (e > -105)  # (mag at most 2^(e + 14))
+    bound = (2.0 ** -20 if K <= 128 else (6 + 5 * K / 128) * 2.0 ** -23) * mag + 2.0 ** -149
+    assert ((C.double() - ref).abs() <= bound)[normal].all()
+
+
 # 256 x 256 tiles (27419 rows) and 128 x 128 or smaller (999) for both products
 @pytest.mark.parametrize("M", [999, 27419])
 @pytest.mark.parametrize("act", [1, 2])
