@@ -487,7 +487,10 @@ __global__ void __launch_bounds__(256) pair_rows_kernel(const float* __restrict_
   const int n = blockIdx.x, tid = threadIdx.x, KG = K / 8;
   auto at = [&](int k) { return transposed ? W[int64_t(k) * ldw + n] : W[int64_t(n) * ldw + k]; };
   float m = 0.f;
-  for (int k = tid; k < K; k += 256) m = fmaxf(m, fabsf(at(k)));
+  for (int k = tid; k < K; k += 256) {
+    const float x = fabsf(at(k));
+    m = fmaxf(m, P == 3 && x > pet_split::kFltMax ? 0.f : x);  // (infinities: pair3)
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
   if ((tid & 63) == 0) red[tid >> 6] = m;

@@ -87,12 +87,56 @@ __device__ __forceinline__ void split8x(u4& x, u4& y, float s) {
 __device__ __forceinline__ float outgrow(float m, float& sa, float& lim) {
   const float rm = max_g(m);
   float f = 1.f;
-  if (rm > lim) {  // (rm finite: infinities are taken out before)
+  if (rm > lim) {  // (an infinity: any scale, special_rows makes the row's results)
     const int k = min(12 - __builtin_amdgcn_frexp_expf(rm), 126);
     f = __builtin_amdgcn_ldexpf(lim, k - 15);
     sa = __builtin_amdgcn_ldexpf(1.f, k), lim = fminf(__builtin_amdgcn_ldexpf(1.f, 15 - k), pet_split::kFltMax);
   }
   return f;
+}
+
+// Rows of A that hold an infinity or a NaN. Split into parts an infinity makes
+// NaN of its row (inf - inf), every column alike; such a row's results are made
+// again after its K loop, on the matrix cores, from its infinities and NaNs
+// alone (no finite value has a say) and the weights' signs: infinite times the
+// weight's sign, NaN against a zero weight or where both signs meet, as fp32
+// gives. A weight's first part carries its sign, unless the weight itself is
+// infinite: then the last (pair3). The check is one ballot a tile; kept in the K
+// loop, where the rows' scales are, it cost 1 to 2% of the model's layers.
+__device__ __forceinline__ unsigned special_half(unsigned x) {
+  const unsigned m = x & 0x7fffffffu;
+  return m < 0x7f800000u ? 0u : (x >> 16 & 0x8000u) | (m > 0x7f800000u ? 0x7e00u : 0x7c00u);
+}
+// acc: the row's tiles; row(c, s): this lane's 8 floats of step s; weight(c, b, s,
+// hi, lo): its parts of tile b.
+template <int TN, class R, class W>
+__device__ __forceinline__ void special_rows(f4 (&acc)[TN], int steps, int c, R&& row, W&& weight) {
+  const bool bad = acc[0][0] != acc[0][0];
+  if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+  // the lane's row and column of a tile, c, past the compiler's sight: the
+  // addresses are made here and not held in registers by the callers' loops
+  asm volatile("" : "+v"(c));
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+    f4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int s = 0; s < steps; ++s) {
+      const u4* p = row(c, s);
+      const u4 x = p[0], y = p[1];
+      const u4 v = {special_half(x[0]) | special_half(x[1]) << 16, special_half(x[2]) | special_half(x[3]) << 16,
+                    special_half(y[0]) | special_half(y[1]) << 16, special_half(y[2]) | special_half(y[3]) << 16};
+      u4 h, lo;
+      weight(c, b, s, h, lo);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const unsigned lh = h[j] & 0x7fffu ? h[j] : lo[j], hh = h[j] & 0x7fff0000u ? h[j] : lo[j];
+        h[j] = (lh & 0xffffu) | (hh & 0xffff0000u);
+      }
+      t = mfma_h(h, v, t);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[b][e] = bad ? t[e] : acc[b][e];
+  }
 }
 
 // A step of 32 is summed from zero and added to the running sum; with three-part
@@ -574,6 +618,18 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   }
   add_group(last_{}, NG - 1);
   wait_vm<0>();  // no load into LDS outlives the loop
+  if constexpr (AS == kOnline)
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+      special_rows(
+          acc[a], steps, c,
+          [&](int c, int s) {
+            return reinterpret_cast<const u4*>(static_cast<const char*>(A) + min(m0 + 16 * a + c, M - 1) * arow + 128 * int64_t(s) + 32 * g);
+          },
+          [&](int c, int b, int s, u4& h, u4& lo) {
+            const u4* q = B + int64_t(min(nt + col_of(bc + 16 * b + c), N - 1)) * KG * P + s * CH + g * P;
+            h = q[0], lo = q[P - 1];
+          });
 
   // ---- epilogue
   float ia[TM];
@@ -706,6 +762,15 @@ gemm_ksplit_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B,
       for (int e = 0; e < 4; ++e) sum[0][b][e] = fmaf(x[e], inv[v] * (1.f / top), sum[0][b][e]);
     }
   }
+  special_rows(
+      sum[0], steps, c,
+      [&](int c, int s) {
+        return reinterpret_cast<const u4*>(static_cast<const char*>(A) + min(m0 + 16 * w + c, M - 1) * (4 * lda) + 128 * int64_t(s) + 32 * g);
+      },
+      [&](int c, int b, int s, u4& h, u4& lo) {
+        const u4* q = B + int64_t(min(n0 + col_of(16 * b + c), N - 1)) * KG * P + s * CH + g * P;
+        h = q[0], lo = q[P - 1];
+      });
   const float ia[1] = {top};
   rows_epilogue<1, TN, OUT, true>(sum, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0 + 16 * w, n0, c, g, M,
                             N, C, ldc, epi);
@@ -839,6 +904,15 @@ gemm_strip_kernel(int M, int N, const float* A, int64_t lda, const u4* B, float*
       }
     }
     add_group(std::integral_constant<int, (G - 1) & 1>{}, G - 1);
+    special_rows(
+        acc[0], KB, c,
+        [&](int c, int s) {
+          return reinterpret_cast<const u4*>(reinterpret_cast<const char*>(A) + min(xr0 + 16 * blk + c, xr1 - 1) * (4 * lda) + 128 * s + 32 * g);
+        },
+        [&](int c, int b, int s, u4& h, u4& lo) {
+          const u4* q = lds + (s * BN + 16 * b + c) * CH;
+          h = q[sb[0]], lo = q[sb[2]];
+        });
     const float ia[1] = {1.f / sa};
     rows_epilogue<1, TN, OUT, true>(acc, ia, inv_b, xr0 + 16 * blk, n0, c, g, xr1, N, C, ldc, epi);
     // the next block's loads done: issued before the epilogue, whose last

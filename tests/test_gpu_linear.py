@@ -731,6 +731,35 @@ def test_three_part_range(M, N, K, device):
     assert ((C.double() - ref).abs() <= bound)[normal].all()
 
 
+@pytest.mark.parametrize("M,N,K", RANGE)
+def test_three_part_infinities(M, N, K, device):
+    """Infinite activations and weights give the infinities and NaNs that IEEE
+    sums of the products do (float64's), and leave the other rows and columns as they
+    are without them, bit for bit."""
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    A = torch.randn(M, K, device=device, generator=g)
+    W = torch.randn(N, K, device=device, generator=g)
+    A[2 % M], A[12 % M] = 0, 0  # rows of nothing else
+    W[N // 2, K - 1] = 0
+    C0, C1 = torch.empty(M, N, device=device), torch.empty(M, N, device=device)
+    L.fused_parts(A, L.PairWeights(W), C0)
+    B = A.clone()
+    inf = float("inf")
+    B[M // 2, 3], B[M // 2, K - 1] = inf, inf  # one sign or both by the weights; zero times infinity
+    B[M - 1, K - 1], B[2 % M, K - 1], B[12 % M, 0] = -inf, -inf, inf
+    V = W.clone()
+    V[N - 1, 1], V[0, K - 2] = -inf, inf
+    for X, Y in ((B, W), (A, V)):
+        L.fused_parts(X, L.PairWeights(Y), C1)
+        ref = X.double().cpu() @ Y.double().cpu().T
+        rows, cols = torch.isfinite(X).all(1), torch.isfinite(Y).all(1)
+        assert torch.equal(C1[rows][:, cols], C0[rows][:, cols])
+        rest = ~(rows[:, None] & cols).cpu()
+        got, want = C1.cpu()[rest].double(), ref[rest]
+        assert not torch.isfinite(want).any()
+        assert torch.equal(got.nan_to_num(-7.0, inf, -inf), want.nan_to_num(-7.0, inf, -inf))
+
+
 # 256 x 256 tiles (27419 rows) and 128 x 128 or smaller (999) for both products
 @pytest.mark.parametrize("M", [999, 27419])
 @pytest.mark.parametrize("act", [1, 2])
