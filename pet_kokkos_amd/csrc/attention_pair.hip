@@ -78,6 +78,7 @@ namespace {
 // us (427 with mfma_block), forward 207 -> 173; S 143 (nine waves) 373 -> 280
 // and 114 -> 100.
 constexpr int kPairMaxWaves = 16;
+constexpr float kFltMax = 3.40282347e38f;
 constexpr int pair_waves(int NW) { return NW <= 9 ? NW : (NW + 1) & ~1; }
 
 struct PairLds {
@@ -182,8 +183,19 @@ __device__ __forceinline__ float row_max16(float x) {
 // The exponent k of the pair scale 2^k that puts m = f 2^e (f in [0.5, 1))
 // at [2^14, 2^15): 15 - e; 0 for a zero (or non-finite) m.
 __device__ __forceinline__ int pair_exp(float m) {
-  if (!(m > 0.f) || m > 3.0e38f) return 0;
+  if (!(m > 0.f) || m > kFltMax) return 0;
   return min(15 - __builtin_amdgcn_frexp_expf(m), 126);
+}
+// The largest finite |x| of n values: the scale of a row whose norm's square
+// passes a float (|x| from 2^64). Past 128 slots only, whose fp32 kernels held
+// such rows; the check there is 1% of both kernels' time (640 atoms of 180
+// neighbours, forward and backward 581 -> 587 us).
+template <int n>
+__device__ __forceinline__ float amax_finite(const float* x) {
+  float m = 0.f;
+#pragma unroll
+  for (int t = 0; t < n; ++t) m = fmaxf(m, fabsf(x[t]) <= kFltMax ? fabsf(x[t]) : 0.f);
+  return m;
 }
 
 // The fused QKV transform (QkvXf: qkv[r][j] rs[r] + b[j]) applied to a lane's
@@ -388,8 +400,35 @@ __device__ __forceinline__ void pair_bwd_item(const PairBwdArgs& a, const Atom& 
   for (int u = 0; u < 5; ++u) M[u] = __builtin_amdgcn_sqrtf(M[u]);  // largest norms, largest |D| (only their exponents matter)
   // scales 2^k: Q, K, V, dO by their largest row norm; dS by its bound
   // |dS_ij| = P_ij |dO_i.v_j - D_i| <= max|v| max|dO| + max|D| (Cauchy-Schwarz, P <= 1)
-  const int kQ = pair_exp(M[0]), kK = pair_exp(M[1]), kV = pair_exp(M[2]), kG = pair_exp(M[3]);
-  const int kS = pair_exp(fmaf(M[2], M[3], M[4]));
+  int kQ = pair_exp(M[0]), kK = pair_exp(M[1]), kV = pair_exp(M[2]), kG = pair_exp(M[3]);
+  int kS = pair_exp(fmaf(M[2], M[3], M[4]));
+  if constexpr (NW > 8) {
+    if (__builtin_expect(!(fmaf(M[2], M[3], M[4]) + (M[0] + M[1]) <= kFltMax), 0)) {  // (the same in every wave: from LDS)
+      // a square past the range: the scales from the largest |x|, dS's from
+      // |dO_i.v_j| < 2^(eV + eG) HD and |D|
+      float m[5] = {max_g(amax_finite<W>(q)), max_g(amax_finite<W>(k)), max_g(amax_finite<W>(v)),
+                    max_g(amax_finite<W>(go)), amax_finite<1>(&Di)};
+      lds_barrier();  // every wave has read the norms
+#pragma unroll
+      for (int u = 0; u < 5; ++u) m[u] = active ? row_max16(m[u]) : 0.f;
+      if (l == 0) {
+#pragma unroll
+        for (int u = 0; u < 5; ++u) red[8 * w + u] = m[u];
+      }
+      lds_barrier();
+#pragma unroll
+      for (int u = 0; u < 5; ++u) {
+        M[u] = 0.f;
+        for (int x = 0; x < NW; ++x) M[u] = fmaxf(M[u], red[8 * x + u]);
+      }
+      kQ = pair_exp(M[0]), kK = pair_exp(M[1]), kV = pair_exp(M[2]), kG = pair_exp(M[3]);
+      int e = -112;
+      if (M[2] > 0.f && M[3] > 0.f)
+        e = max(e, __builtin_amdgcn_frexp_expf(M[2]) + __builtin_amdgcn_frexp_expf(M[3]) + (HD > 32 ? 6 : 5));
+      if (M[4] > 0.f) e = max(e, __builtin_amdgcn_frexp_expf(M[4]));
+      kS = 14 - e;
+    }
+  }
   constexpr int kP = 15;  // P's scale 2^15
   const float sQ = __builtin_amdgcn_ldexpf(1.f, kQ), sK = __builtin_amdgcn_ldexpf(1.f, kK);
   const float sV = __builtin_amdgcn_ldexpf(1.f, kV), sG = __builtin_amdgcn_ldexpf(1.f, kG);
@@ -685,9 +724,19 @@ attn_fwd_pair_kernel(const float* __restrict__ qkv, int64_t ldq, const int* __re
   float nq = 0.f, nk = 0.f, nv = 0.f;
 #pragma unroll
   for (int t = 0; t < W; ++t) nq = fmaf(q[t], q[t], nq), nk = fmaf(k[t], k[t], nk), nv = fmaf(v[t], v[t], nv);
-  const int kQ = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(row_max16(sum_g(nq)))));
-  const int kKw = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(row_max16(sum_g(nk)))));
-  const int kVw = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(row_max16(sum_g(nv)))));
+  const float mq = row_max16(sum_g(nq)), mk = row_max16(sum_g(nk)), mv = row_max16(sum_g(nv));
+  int kQ = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(mq)));
+  int kKw = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(mk)));
+  int kVw = __builtin_amdgcn_readfirstlane(pair_exp(__builtin_amdgcn_sqrtf(mv)));
+  bool wide = false;
+  if constexpr (NW > 8) {  // a square past the range: the scales from the largest |x|
+    wide = __builtin_amdgcn_ballot_w64(!(mq + mk + mv <= kFltMax)) != 0;
+    if (__builtin_expect(wide, 0)) {
+      kQ = __builtin_amdgcn_readfirstlane(pair_exp(row_max16(max_g(amax_finite<W>(q)))));
+      kKw = __builtin_amdgcn_readfirstlane(pair_exp(row_max16(max_g(amax_finite<W>(k)))));
+      kVw = __builtin_amdgcn_readfirstlane(pair_exp(row_max16(max_g(amax_finite<W>(v)))));
+    }
+  }
   if (l == 0) kex[2 * w] = kKw, kex[2 * w + 1] = kVw;
   if (g == 0) lcf[i] = pcf > 0.f ? log_cf(pcf) : kOff;
   const float sQ = __builtin_amdgcn_ldexpf(1.f, kQ), sK = __builtin_amdgcn_ldexpf(1.f, kKw);
@@ -710,6 +759,18 @@ attn_fwd_pair_kernel(const float* __restrict__ qkv, int64_t ldq, const int* __re
       const int o = tok_off<HD, true>(i, 4 * kc + g);
       *reinterpret_cast<u4*>(KTh + o) = kp[0], *reinterpret_cast<u4*>(KTh + PS + o) = kp[1];
       *reinterpret_cast<u4*>(VTh + o) = vp[0], *reinterpret_cast<u4*>(VTh + PS + o) = vp[1];
+    }
+  }
+  if constexpr (NW > 8) {
+    if (__builtin_expect(wide, 0) && active) {
+      // an infinite v: in the lo part alone, which meets only the weights' hi
+      // parts, none negative: infinite in its dim, as fp32 gives
+#pragma unroll
+      for (int x = 0; x < W; ++x)
+        if (fabsf(v[x]) > kFltMax) {
+          const int o = tok_off<HD, true>(i, 4 * (x >> 3) + g) + (x & 7);
+          VTh[o] = _Float16(0.f), VTh[PS + o] = _Float16(v[x]);
+        }
     }
   }
   if (!active) {  // slots past the atom's tokens: their sentinel statistics, and the workgroup barrier

@@ -139,6 +139,42 @@ def test_pair_kernels_past_128_slots(device, hd, S):
     check_against_oracle(device, f"pair kernels S {S} hd {hd}", tk.off, tk.cf_seq, qkv, dm, 2, hd)
 
 
+@pytest.mark.parametrize("hd,S", [(32, 129), (32, 200), (32, 256), (64, 150)])
+@pytest.mark.parametrize("which,e", [("v", 84), ("v", 110), ("dO", 70), ("dO", 110), ("q", 70), ("one v", 80)])
+def test_pair_kernels_past_128_slots_range(device, hd, S, which, e):
+    # values whose squares pass a float (from 2^64), as the fp32 kernels that these
+    # shapes had took them: V, dO, Q against as small a K, and one token's V alone
+    H, D = 2, 2 * hd
+    tk, qkv, dm = random_case([S - 1, S // 2, 140, 1], H, hd, seed=S + e)
+    big = np.float32(2.0 ** e)
+    if which == "v":
+        qkv[:, 2 * D:] *= big
+    elif which == "one v":
+        qkv[2, 2 * D:] *= big
+    elif which == "q":
+        qkv[:, :D] *= big
+        qkv[:, D:2 * D] /= big
+    else:
+        dm *= big
+    check_against_oracle(device, f"{which} 2^{e} S {S} hd {hd}", tk.off, tk.cf_seq, qkv, dm, H, hd)
+
+
+@pytest.mark.parametrize("hd,S", [(32, 129), (32, 200), (32, 256), (64, 150), (64, 250)])
+def test_pair_kernels_past_128_slots_infinite_value(device, hd, S):
+    # an infinite V is infinite in its own dim of its atom's rows and nowhere else
+    H, D = 2, 2 * hd
+    tk, qkv, _ = random_case([140, S - 1, 130], H, hd, seed=S)
+    off, cf = dev(tk.off, device, torch.int32), dev(tk.cf_seq, device)
+    clean, _ = A.attn_fwd(dev(qkv, device), off, cf, H, hd)
+    edge = tk.n_atoms + int(tk.off[1]) + S // 2  # an edge's token of atom 1
+    qkv[edge, 2 * D + hd + 3] = -np.inf
+    got, _ = A.attn_fwd(dev(qkv, device), off, cf, H, hd)
+    rows = [1] + list(range(tk.n_atoms + int(tk.off[1]), tk.n_atoms + int(tk.off[2])))
+    assert torch.equal(got[rows, hd + 3], torch.full((len(rows),), -float("inf"), device=device))
+    got[rows, hd + 3] = clean[rows, hd + 3]
+    assert row_err(got.cpu().numpy(), clean.cpu().numpy()) <= RTOL
+
+
 @pytest.mark.parametrize("S,hd", [(143, 32), (220, 32), (150, 64)])
 def test_op_level_block_pairs_past_128_slots(device, S, hd):
     # qkv_adj as block pairs into the input adjoint's product, past eight
