@@ -9,6 +9,8 @@
 // orders so the bits repeat from run to run.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <cstdint>
 
 #include "../../include/pet_attn.h"
@@ -114,56 +116,90 @@ __global__ void edge_grad_kernel(int nc, int E, const int* __restrict__ off, con
   for (int c = 0; c < 3; ++c) g[c] = double(xa[c]) + dist_adj * v[c] * invd;
 }
 
+// An atom's forces and virial by one thread, its edges in order: the reference's
+// sums exactly.
+__device__ __forceinline__ void fold_thread(int i, int nc, const int* __restrict__ off, const int* __restrict__ rev,
+                                            const double* __restrict__ vec, const double* __restrict__ grad,
+                                            double scale, double* __restrict__ forces, double* __restrict__ vir) {
+  double f[3] = {0.0, 0.0, 0.0}, w[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  const int k0 = i < nc ? off[i] : 0, k1 = i < nc ? off[i + 1] : 0;
+  for (int k = k0; k < k1; ++k) {
+    const double g0 = grad[3 * int64_t(k)], g1 = grad[3 * int64_t(k) + 1], g2 = grad[3 * int64_t(k) + 2];
+    const double v0 = vec[3 * int64_t(k)], v1 = vec[3 * int64_t(k) + 1], v2 = vec[3 * int64_t(k) + 2];
+    f[0] += g0, f[1] += g1, f[2] += g2;
+    w[0] += v0 * g0, w[1] += v0 * g1, w[2] += v0 * g2;
+    w[3] += v1 * g0, w[4] += v1 * g1, w[5] += v1 * g2;
+    w[6] += v2 * g0, w[7] += v2 * g1, w[8] += v2 * g2;
+    const int r = rev[k];
+    if (r >= 0) f[0] -= grad[3 * int64_t(r)], f[1] -= grad[3 * int64_t(r) + 1], f[2] -= grad[3 * int64_t(r) + 2];
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) forces[3 * int64_t(i) + c] = scale * f[c];
+  if (vir)
+#pragma unroll
+    for (int t = 0; t < 9; ++t) vir[9 * int64_t(i) + t] = scale * w[t];
+}
+
 // A wavefront an atom: its lanes load 64 edges' gradients, reverse gradients
 // and vectors at once and leave them in LDS, and 12 lanes (three forces, nine
-// virial entries) each add theirs edge by edge in the list's order -- the
-// reference's sums exactly. One thread an atom walking its edges waited on
-// memory once an edge, with seven workgroups on the device: 60 us for 1728
-// atoms of 70 edges and 36 us for 192 atoms of 41; this form takes 10.5 and
-// 5.8 us (MI355X, kernel trace), the same bits.
+// virial entries) each add theirs edge by edge in the list's order, the same
+// sums. A thread an atom waits on memory once an edge: 60 us for 1728 atoms of
+// 70 edges and 36 us for 192 atoms of 41; the wavefronts take 10.5 and 5.8 us
+// (MI355X, kernel trace), the same bits. With few edges an atom and atoms
+// enough, threads are faster (16000 atoms of 2 edges 3.7 us against 7.4; 64000
+// of 8 19 against 33, of 16 39 against 43, of 32 84 against 71): from kFoldThreads
+// atoms with at most 12 edges on the mean, which the kernel reads off the list.
+// The grid is bounded and strides over the atoms, so any count of them fits.
 constexpr int kFoldPitch = 65;  // doubles: the 12 lanes' rows of a chunk on distinct banks
+constexpr int kFoldThreads = 8192, kFoldBlocks = 2048;  // (eight workgroups a CU by their LDS)
 __global__ void __launch_bounds__(256) fold_kernel(int N, int nc, const int* __restrict__ off,
                                                    const int* __restrict__ rev, const double* __restrict__ vec,
                                                    const double* __restrict__ grad, double scale,
                                                    double* __restrict__ forces, double* __restrict__ vir) {
   __shared__ double sh[4][9 * kFoldPitch];  // a wave's chunk: gradient | reverse gradient | vector, 3 rows each
-  const int i = blockIdx.x * 4 + int(threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (N >= kFoldThreads && (nc == 0 || int64_t(off[nc]) - off[0] <= 12 * int64_t(nc))) {
+    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256)
+      fold_thread(int(i), nc, off, rev, vec, grad, scale, forces, vir);
+    return;
+  }
+  const int l = threadIdx.x & 63;
   double* x = sh[threadIdx.x >> 6];
-  const int k0 = i < nc ? off[i] : 0, k1 = i < nc ? off[i + 1] : 0;
   // lane 0 .. 2: force component l; 3 .. 11: virial entry l - 3 = 3 a + b
   const int t = l < 3 ? 0 : l < 12 ? l - 3 : 0;
   const double* gp = x + (l < 3 ? l : t % 3) * kFoldPitch;      // g_l, g_b
   const double* rp = x + (l < 3 ? 3 + l : 6 + t / 3) * kFoldPitch;  // the reverse edge's g_l, v_a
-  double s = 0.0;
-  for (int c = k0; c < k1; c += 64) {
-    const int k = c + l;
-    if (k < k1) {
-      const int r = rev[k];
+  for (int64_t i = blockIdx.x * 4 + int(threadIdx.x >> 6); i < N; i += gridDim.x * 4) {
+    const int k0 = i < nc ? off[i] : 0, k1 = i < nc ? off[i + 1] : 0;
+    double s = 0.0;
+    for (int c = k0; c < k1; c += 64) {
+      const int k = c + l;
+      if (k < k1) {
+        const int r = rev[k];
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        x[d * kFoldPitch + l] = grad[3 * int64_t(k) + d];
-        x[(3 + d) * kFoldPitch + l] = r >= 0 ? grad[3 * int64_t(r) + d] : 0.0;
-        x[(6 + d) * kFoldPitch + l] = vec[3 * int64_t(k) + d];
+        for (int d = 0; d < 3; ++d) {
+          x[d * kFoldPitch + l] = grad[3 * int64_t(k) + d];
+          x[(3 + d) * kFoldPitch + l] = r >= 0 ? grad[3 * int64_t(r) + d] : 0.0;
+          x[(6 + d) * kFoldPitch + l] = vec[3 * int64_t(k) + d];
+        }
       }
-    }
-    // LDS operations of one wave complete in order: no barrier, the fences
-    // only keep the compiler from moving the accesses across them
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const int n = k1 - c < 64 ? k1 - c : 64;
-    if (l < 3) {
+      // LDS operations of one wave complete in order: no barrier, the fences
+      // only keep the compiler from moving the accesses across them
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int n = k1 - c < 64 ? k1 - c : 64;
+      if (l < 3) {
 #pragma unroll 8
-      for (int k = 0; k < n; ++k) s += gp[k], s -= rp[k];
-    } else if (l < 12) {
+        for (int k = 0; k < n; ++k) s += gp[k], s -= rp[k];
+      } else if (l < 12) {
 #pragma unroll 8
-      for (int k = 0; k < n; ++k) s += rp[k] * gp[k];
+        for (int k = 0; k < n; ++k) s += rp[k] * gp[k];
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (l < 3) forces[3 * i + l] = scale * s;
+    else if (l < 12 && vir) vir[9 * i + t] = scale * s;
   }
-  if (i >= N) return;
-  if (l < 3) forces[3 * int64_t(i) + l] = scale * s;
-  else if (l < 12 && vir) vir[9 * int64_t(i) + t] = scale * s;
 }
 
 // A wavefront per (structure, column): lane l sums atoms a0 + l, a0 + l + 64,
@@ -221,7 +257,7 @@ int pet_fold_edge_gradients(int n_atoms, int n_centres, const int* off, const in
   if (n_atoms < 0 || n_centres < 0 || n_centres > n_atoms) return PET_ATTN_EINVAL;
   if (n_atoms == 0) return PET_ATTN_OK;
   if (!forces || (n_centres > 0 && (!off || !reverse || !vec || !grad))) return PET_ATTN_EINVAL;
-  hipLaunchKernelGGL(fold_kernel, dim3(unsigned((n_atoms + 3) / 4)), dim3(256), 0,
+  hipLaunchKernelGGL(fold_kernel, dim3(unsigned(std::min((int64_t(n_atoms) + 3) / 4, int64_t(kFoldBlocks)))), dim3(256), 0,
                      reinterpret_cast<hipStream_t>(stream), n_atoms, n_centres, off, reverse, vec, grad, scale, forces,
                      virial_atom);
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;

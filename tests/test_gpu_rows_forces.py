@@ -145,6 +145,52 @@ def test_edge_grad_dead_rows_and_neighbour_only_atoms(device):
     assert np.all(forces.cpu().numpy()[N:] == 0.0) and np.all(vir.cpu().numpy()[N:] == 0.0)
 
 
+@pytest.mark.parametrize("N", [8191, 8192, 20011])
+@pytest.mark.parametrize("mean", [0, 2, 11, 12, 13, 30])
+def test_fold_threads_and_wavefronts(device, N, mean):
+    """Either side of the rule by which an atom is folded by a thread or by a
+    wavefront (8192 atoms, 12 edges on the mean), with a few atoms far above the
+    mean; in the oracle's order, as test_fold_chunks_of_edges."""
+    rng = np.random.default_rng(N + mean)
+    counts = np.full(N, mean)
+    counts[: N // 2] -= min(mean, 3)
+    counts[N // 2: 2 * (N // 2)] += min(mean, 3)
+    if mean <= 2:
+        counts[::1000] = 200 if mean else 1
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    E = int(off[-1])
+    vec, g = rng.standard_normal((E, 3)), rng.standard_normal((E, 3))
+    rev = rng.integers(-1, E, E).astype(np.int32)
+    center = np.repeat(np.arange(N), counts).astype(np.int32)
+    one = np.ones(E)
+    dpk = F.PackedEdges.from_host(systems.PackedEdges(off, center, center, rev, vec, one, one, one.astype(np.float32)),
+                                  device)
+    forces, vir = F.fold_edge_gradients(dpk, N + 7, dev(g, device), scale=0.5)
+    rf, rv = oracle.fold(N, off, rev, vec, g, scale=0.5)
+    forces, vir = forces.cpu().numpy(), vir.cpu().numpy()
+    assert not forces[N:].any() and not vir[N:].any()
+    assert np.abs(forces[:N] - rf).max(initial=0) <= 1e-12 * np.abs(rf).max(initial=0)
+    assert np.abs(vir[:N] - rv).max(initial=0) <= 1e-12 * np.abs(rv).max(initial=0)
+
+
+@pytest.mark.parametrize("edges", [2, 40])
+def test_fold_more_atoms_than_a_grid_of_wavefronts(device, edges):
+    """2^26 atoms and three, a wavefront each, are more threads than a launch
+    holds; two of them are centres."""
+    N = 2 ** 26 + 3
+    print(f"[gpu] fold {N} atoms", flush=True)
+    g = torch.arange(3 * 2 * edges, device=device, dtype=torch.float64).reshape(-1, 3)
+    off = torch.tensor([0, edges, 2 * edges], device=device, dtype=torch.int32)
+    rev = torch.full((2 * edges,), -1, device=device, dtype=torch.int32)
+    one = torch.ones(2 * edges, device=device, dtype=torch.float64)
+    dpk = F.PackedEdges(off, torch.zeros_like(rev), rev, torch.ones_like(g), one, one)
+    forces, vir = F.fold_edge_gradients(dpk, N, g)
+    for i in (0, 1):
+        f = g[i * edges:(i + 1) * edges].sum(0)
+        assert torch.equal(forces[i], f) and torch.equal(vir[i], f.repeat(3))
+    assert not forces[2:].any() and not vir[2:].any()
+
+
 @pytest.mark.parametrize("counts", [[0, 1, 63, 0], [64, 65, 127], [128, 129, 2, 300]])
 def test_fold_chunks_of_edges(device, counts):
     """Atoms with no edge, and edge counts around the 64 a wavefront takes at
