@@ -248,25 +248,26 @@ __global__ void __launch_bounds__(256) readout_kernel(float* __restrict__ net, c
                                                       const int* __restrict__ off, const float* __restrict__ cut,
                                                       int acc, int N) {
   __shared__ double sh[4][64];
-  const int n = blockIdx.x * 4 + int(threadIdx.x >> 6), l = threadIdx.x & 63;
-  if (n >= N) return;
+  const int l = threadIdx.x & 63;
   double* x = sh[threadIdx.x >> 6];
-  double s = node_pred[n];
-  const int k1 = off[n + 1];
-  for (int c = off[n]; c < k1; c += 64) {
-    if (c + l < k1) x[l] = double(cut[c + l]) * double(edge_pred[c + l]);
-    // one wave's LDS operations complete in order: only the compiler is fenced
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const int m = k1 - c < 64 ? k1 - c : 64;
-    if (l == 0) {
+  for (int64_t n = int64_t(blockIdx.x) * 4 + int(threadIdx.x >> 6); n < N; n += int64_t(gridDim.x) * 4) {
+    double s = node_pred[n];
+    const int k1 = off[n + 1];
+    for (int c = off[n]; c < k1; c += 64) {
+      if (c + l < k1) x[l] = double(cut[c + l]) * double(edge_pred[c + l]);
+      // one wave's LDS operations complete in order: only the compiler is fenced
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int m = k1 - c < 64 ? k1 - c : 64;
+      if (l == 0) {
 #pragma unroll 8
-      for (int k = 0; k < m; ++k) s += x[k];
+        for (int k = 0; k < m; ++k) s += x[k];
+      }
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (l == 0) net[n] = acc ? float(double(net[n]) + s) : float(s);
   }
-  if (l == 0) net[n] = acc ? float(double(net[n]) + s) : float(s);
 }
 
 // per_atom = scale * net + composition[species] (assemble_energy, src/ops.cpp:420-425)
@@ -1329,7 +1330,9 @@ struct Pass {
     linear(md, r.epred, y, E, Dh, "edge_last_layers.energy." + si + ".energy___0", st);
     md.ws.release(scope);
     if (N) {
-      hipLaunchKernelGGL(readout_kernel, dim3(unsigned((N + 3) / 4)), dim3(256), 0, st, net, r.npred, r.epred,
+      // (a bounded grid: a launch holds fewer than 2^32 threads)
+      const int64_t blocks = std::min((int64_t(N) + 3) / 4, int64_t(1) << 20);
+      hipLaunchKernelGGL(readout_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, net, r.npred, r.epred,
                          e.off, e.cut, acc ? 1 : 0, N);
       launched();
     }
