@@ -474,14 +474,36 @@ __global__ void split_rows_kernel(const float* __restrict__ W, int N, int K, int
   for (int p = 0; p < 3; ++p) out[t * 3 + p] = parts[p];
 }
 
+// pair2's lo parts of x and y with their ties (a remainder halfway between two
+// fp16 numbers: every fourth weight) broken so that the errors of a group of
+// eight, summed in carry, cancel: the same in every product with the weight, they
+// add up over a structure (eight 648-atom structures on a 512-wide model 3.7e-6 eV
+// an atom (rms) from float64 with ties to even, 3.0e-6 so).
+__device__ __forceinline__ unsigned even_ties(float x, float y, unsigned hi, unsigned lo, float& carry) {
+  const pet_split::h2v h = __builtin_bit_cast(pet_split::h2v, hi);
+  pet_split::h2v l = __builtin_bit_cast(pet_split::h2v, lo);
+  const float v[2] = {x, y};
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float err = v[e] - float(h[e]) - float(l[e]), other = float(l[e]) + 2.f * err;
+    const bool flip = err * carry > 0.f && float(_Float16(other)) == other;
+    carry += flip ? -err : err;
+    if (flip) l[e] = _Float16(other);
+  }
+  return __builtin_bit_cast(unsigned, l);
+}
+
 // Rows of B = W (transposed false: W [N, K], ld ldw) or B = W^T (transposed
 // true: W [K, N]) as P fp16 parts: out[(n K/8 + j) P + p] = part p of row n's
 // k group j, scaled by the row's s_n (P 2: hi and lo, pair2; P 3: hi, mid and
 // lo, pair3, W exactly); then at byte N K 2 P the N inverse scales 1 / s_n.
+// alt (P 2): the values of odd steps of 32 negated, and the inverse scales too, which
+// tells the product that reads them (gemm_rows.hip, add_step) to subtract
+// those steps' sums; lo's ties by even_ties.
 // One workgroup a row: its largest |x|, then its groups.
 template <int P>
 __global__ void __launch_bounds__(256) pair_rows_kernel(const float* __restrict__ W, int N, int K, int64_t ldw,
-                                                         bool transposed, u4* __restrict__ out) {
+                                                         bool transposed, bool alt, u4* __restrict__ out) {
   static_assert(P == 2 || P == 3, "two or three parts");
   __shared__ float red[4];
   const int n = blockIdx.x, tid = threadIdx.x, KG = K / 8;
@@ -498,12 +520,15 @@ __global__ void __launch_bounds__(256) pair_rows_kernel(const float* __restrict_
   const float s = pair_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
   for (int j = tid; j < KG; j += 256) {
     u4 pt[P];
+    float carry = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float x = at(8 * j + 2 * e) * s, y = at(8 * j + 2 * e + 1) * s;
+      const float sj = alt && (j & 4) ? -s : s;
+      const float x = at(8 * j + 2 * e) * sj, y = at(8 * j + 2 * e + 1) * sj;
       unsigned h, md, lw;
       if constexpr (P == 2) {
         pair2(x, y, h, lw);
+        if (alt) lw = even_ties(x, y, h, lw, carry);
         pt[0][e] = h, pt[1][e] = lw;
       } else {
         pet_split::pair3(x, y, h, md, lw);
@@ -513,7 +538,7 @@ __global__ void __launch_bounds__(256) pair_rows_kernel(const float* __restrict_
 #pragma unroll
     for (int p = 0; p < P; ++p) out[(int64_t(n) * KG + j) * P + p] = pt[p];
   }
-  if (tid == 0) reinterpret_cast<float*>(out + int64_t(N) * KG * P)[n] = 1.f / s;
+  if (tid == 0) reinterpret_cast<float*>(out + int64_t(N) * KG * P)[n] = (alt ? -1.f : 1.f) / s;
 }
 
 // Rows of an activation X [M, K] (ld ldx) as fp16 pairs in pair_rows_kernel's
@@ -768,13 +793,16 @@ int pet_gemm_nt_split_f32b(int M, int N, int K, const float* A, int64_t lda, con
 }
 
 // B [N, K] as split rows, from W = B (transposed false: W [N, K]) or W = B^T
-// (transposed true: W [K, N]); K a multiple of 32, out 16-byte aligned.
-int pet_gemm_split_weights(const float* W, int N, int K, int64_t ldw, bool transposed, void* out, hipStream_t st) {
+// (transposed true: W [K, N]); K a multiple of 32, out 16-byte aligned. alt: pairs
+// with steps of either sign (pair_rows_kernel), for the products of a model and
+// of the layer level, whose errors' mean adds up over a structure's atoms.
+int pet_gemm_split_weights(const float* W, int N, int K, int64_t ldw, bool transposed, bool alt, void* out,
+                           hipStream_t st) {
   if (N < 0 || K < 0 || K % 32 || (reinterpret_cast<uintptr_t>(out) & 15)) return PET_ATTN_EINVAL;
   const int64_t n = int64_t(N) * (K / 8);
   if (n == 0) return PET_ATTN_OK;
   if (pair_form(K))
-    hipLaunchKernelGGL(pair_rows_kernel<2>, dim3(unsigned(N)), dim3(256), 0, st, W, N, K, ldw, transposed,
+    hipLaunchKernelGGL(pair_rows_kernel<2>, dim3(unsigned(N)), dim3(256), 0, st, W, N, K, ldw, transposed, alt,
                        static_cast<u4*>(out));
   else if (transposed)
     hipLaunchKernelGGL(split_rows_t_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, W, N, K, ldw,
@@ -790,14 +818,14 @@ extern "C" int pet_linear_split_weights(const float* W, int N, int K, int64_t ld
   if (reinterpret_cast<uintptr_t>(out) & 15) return PET_ATTN_EALIGN;
   const int64_t n = int64_t(N) * (K / 8);
   if (n == 0) return PET_ATTN_OK;
-  return pet_gemm_split_weights(W, N, K, ldw, false, out, reinterpret_cast<hipStream_t>(stream));
+  return pet_gemm_split_weights(W, N, K, ldw, false, false, out, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int pet_linear_split_weights_transposed(const float* W, int N, int K, int64_t ldw, void* out,
                                                    void* stream) {
   if (N < 0 || K < 0 || K % 32 || ldw < N || ((N > 0 && K > 0) && (!W || !out))) return PET_ATTN_EINVAL;
   if (reinterpret_cast<uintptr_t>(out) & 15) return PET_ATTN_EALIGN;
-  return pet_gemm_split_weights(W, N, K, ldw, true, out, reinterpret_cast<hipStream_t>(stream));
+  return pet_gemm_split_weights(W, N, K, ldw, true, false, out, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int pet_linear_fused_split(int M, int N, int K, const float* A, int64_t lda, const void* Wsplit, float* C,
@@ -893,7 +921,7 @@ int pet_gemm_nt_pp_blocks(int M, int N, int K, const void* Ap, int kb, const voi
 int pet_gemm_pair_weights(const float* W, int N, int K, int64_t ldw, bool transposed, void* out, hipStream_t st) {
   if (N < 0 || K < 0 || K % 32 || (reinterpret_cast<uintptr_t>(out) & 15)) return PET_ATTN_EINVAL;
   if (N == 0 || K == 0) return PET_ATTN_OK;
-  hipLaunchKernelGGL(pair_rows_kernel<3>, dim3(unsigned(N)), dim3(256), 0, st, W, N, K, ldw, transposed,
+  hipLaunchKernelGGL(pair_rows_kernel<3>, dim3(unsigned(N)), dim3(256), 0, st, W, N, K, ldw, transposed, false,
                      static_cast<u4*>(out));
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;
 }

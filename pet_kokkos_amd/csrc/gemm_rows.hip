@@ -145,7 +145,10 @@ __device__ __forceinline__ void special_rows(f4 (&acc)[TN], int steps, int c, R&
 // minus infinity: summed in place, an error of 1.6e-7 (K 128) to 3.2e-7 (K 512) of
 // a result with a mean of -1.6e-8 to -3.3e-8 that a model sums over its atoms
 // (random operands on MI355X; the fp32 matrix core 2.6e-7 to 5.1e-7, mean 0). So it
-// is 0.9e-7 to 1.3e-7, and the steps of either sign cancel the mean.
+// is 0.9e-7 to 1.3e-7, and the steps of either sign cancel the mean. Two-part
+// weights come with their odd steps negated where the mean adds up (their
+// inverse scales are negative then): the energies of 64 structures on a 512-wide
+// model are 5.4e-6 eV an atom (rms) from float64, 9.3e-6 with steps of one sign.
 __device__ __forceinline__ void add_step(f4& acc, const f4& t, float sg) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc[e] = fmaf(t[e], sg, acc[e]);
@@ -300,7 +303,7 @@ __device__ __forceinline__ void rows_epilogue(const f4 (&acc)[TM][TN], const flo
           const bool live = in && i < M;
           float u[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) u[e] = v[e][r] * ib[e];
+          for (int e = 0; e < 4; ++e) u[e] = v[e][r] * fabsf(ib[e]);  // (the sign: add_step)
           if (afar) {
             const int f = far;
             const float p = (r == 0 ? quad_lane<0>(f) : r == 1 ? quad_lane<1>(f) : r == 2 ? quad_lane<2>(f) : quad_lane<3>(f)) ? 0x1p64f : 1.f;
@@ -449,6 +452,11 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   for (int a = 0; a < TM; ++a)
 #pragma unroll
     for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
+  // the sign of odd steps' sums (add_step): the rows are split with it (three
+  // parts), or the weights were
+  const float* inv_b = reinterpret_cast<const float*>(B + int64_t(N) * KG * P);
+  unsigned alt = 0x80000000u;
+  if constexpr (P == 2) alt &= __builtin_amdgcn_readfirstlane(__float_as_uint(inv_b[min(nt, N - 1)]));
   // the row's scale and the largest |x| it takes (kOnline), 1 / scale at the end
   float sa[TM], lim[TM], sg = 1.f;
   // kPairs: the row's largest inverse scale (as its exponent field, a byte a row:
@@ -544,14 +552,16 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
     if constexpr (NG > 1) read(c1_{}, 1);
     __builtin_amdgcn_sched_barrier(0);
     if (s) add_group(last_{}, NG - 1);
-    if constexpr (P == 3) sg = s & 1 ? -1.f : 1.f;
+    sg = __uint_as_float(0x3f800000u | (s & 1 ? alt : 0u));
     if constexpr (AS == kPairs) {
+#pragma unroll
+      for (int a = 0; a < TM; ++a) fac[a] = copysignf(fac[a], sg);
       if (kbs < steps) {
         if (left == 0) {  // a block begins: its factor, and the next one's scale on its way
           left = kbs, blk = min(blk + 1, steps / kbs - 1);
 #pragma unroll
           for (int a = 0; a < TM; ++a) {
-            fac[a] = inext[a] * __uint_as_float((254 - (imax >> (8 * a) & 255)) << 23);
+            fac[a] = sg * inext[a] * __uint_as_float((254 - (imax >> (8 * a) & 255)) << 23);
             inext[a] = inv_a[int64_t(blk) * M + min(m0 + 16 * a + c, M - 1)];
           }
         }
@@ -635,8 +645,7 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   float ia[TM];
 #pragma unroll
   for (int a = 0; a < TM; ++a) ia[a] = AS == kPairs ? __uint_as_float((imax >> (8 * a) & 255) << 23) : 1.f / sa[a];
-  rows_epilogue<TM, TN, OUT, P == 3 || OUT == kBlocks>(acc, ia, reinterpret_cast<const float*>(B + int64_t(N) * KG * P), m0, n0, c, g, M, N, C,
-                             ldc, epi);
+  rows_epilogue<TM, TN, OUT, P == 3 || OUT == kBlocks>(acc, ia, inv_b, m0, n0, c, g, M, N, C, ldc, epi);
 }
 
 // The same product with K split over a workgroup's waves, for launches of few

@@ -46,6 +46,8 @@ int pet_gemm_nt_split(int M, int N, int K, const float* A, int64_t lda, const vo
                       const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
                       float* pre, int64_t ldpre, int act, hipStream_t st, void* scratch = nullptr,
                       size_t scratch_bytes = 0);
+int pet_gemm_split_weights(const float* W, int N, int K, int64_t ldw, bool transposed, bool alt, void* out,
+                           hipStream_t st);
 
 // gemm.hip: block pairs out of one product, into the next
 int pet_gemm_nt_split_pairs(int M, int N, int K, const float* A, int64_t lda, const void* Bs, void* pout,
@@ -1783,7 +1785,7 @@ int pet_model_create(const pet_model_hypers* hy, const pet_model_tensor* tensors
       if (hipMalloc(&md->wsplit, stotal) != hipSuccess) throw Error{PET_MODEL_EMEMORY};
       for (auto& [mt, o] : sat) {
         void* dst = static_cast<char*>(md->wsplit) + o;
-        ok(pet_linear_split_weights(mt->p, mt->rows, mt->cols, mt->cols, dst, nullptr));
+        ok(pet_gemm_split_weights(mt->p, mt->rows, mt->cols, mt->cols, false, true, dst, nullptr));
         md->split[mt->p] = dst;
       }
       if (hipDeviceSynchronize() != hipSuccess) throw Error{PET_ATTN_ELAUNCH};

@@ -18,7 +18,8 @@ int pet_gemm_nt_split(int M, int N, int K, const float* A, int64_t lda, const vo
                       const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
                       float* pre, int64_t ldpre, int act, hipStream_t st, void* scratch = nullptr,
                       size_t scratch_bytes = 0);
-int pet_gemm_split_weights(const float* W, int N, int K, int64_t ldw, bool transposed, void* out, hipStream_t st);
+int pet_gemm_split_weights(const float* W, int N, int K, int64_t ldw, bool transposed, bool alt, void* out,
+                           hipStream_t st);
 int pet_gemm_nt_pp_blocks(int M, int N, int K, const void* Ap, int kb, const void* Bs, float* C, int64_t ldc,
                           const float* row_scale, const float* bias, const float* cin, int64_t ldcin, float beta,
                           float* pre, int64_t ldpre, int act, hipStream_t st);
@@ -94,7 +95,7 @@ int split_dense(float* out, int64_t ldo, const float* A, int64_t lda, const floa
   if (!split || K % 32 || lda % 4 || (reinterpret_cast<uintptr_t>(A) & 15)) return -1;
   const float* cin = beta != 0.f ? out : nullptr;
   if (mnk >= 4294967296.0) {
-    if (int e = pet_gemm_split_weights(W, N, K, ldw, W_is_bt, split, st)) return e;
+    if (int e = pet_gemm_split_weights(W, N, K, ldw, W_is_bt, true, split, st)) return e;
     return pet_gemm_nt_split(M, N, K, A, lda, split, out, ldo, nullptr, bias, cin, ldo, beta, nullptr, 0, 0, st);
   }
   if (!parts || mnk < 134217728.0) return -1;
@@ -264,7 +265,7 @@ int attention_bwd_xf(const pet_attn_shape* sh, float* in_adj, int64_t ldi, int d
     const int rc = pet_attn_bwd_xf_blocks(sh, qkv, ldq, rs, b, off, dmerged, D, merged, D, ml, cf_seq, ldc, qkv_adj,
                                           cfh, cf_seq_adj, ldca, st);
     if (rc == PET_ATTN_OK) {
-      if (int e = pet_gemm_split_weights(w_in, d_in, 3 * D, d_in, true, split_in_t, st)) return e;
+      if (int e = pet_gemm_split_weights(w_in, d_in, 3 * D, d_in, true, true, split_in_t, st)) return e;
       return pet_gemm_nt_pp_blocks(T, d_in, 3 * D, qkv_adj, sh->head_dim, split_in_t, in_adj, ldi, nullptr, nullptr,
                                    beta != 0.f ? in_adj : nullptr, ldi, beta, nullptr, 0, 0, st);
     }
