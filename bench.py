@@ -40,7 +40,7 @@ PEAK_PAIR_FP32 = PEAK_BF16_MFMA / 3
 # the same on the 16x16x16 fp16 instruction, which issues at half the 16x16x32
 # one's FLOP rate (measured on MI355X: 703 against 1236 TFLOP/s at best)
 PEAK_PAIR16_FP32 = PEAK_BF16_MFMA / 2 / 3
-# the short-K dense kernel: an fp32 product as five fp16 products (the
+# the three-part dense kernels: an fp32 product as five fp16 products (the
 # weights in three parts, A in two)
 PEAK_SHORTK_FP32 = PEAK_BF16_MFMA / 5
 PEAK_HBM = 8.0e12  # B/s
@@ -51,7 +51,7 @@ def mixed_seconds(flops, split_share, pair_share=0.0, pair16_share=0.0, shortk_s
     split_share of the FLOPs as split-fp32 products on the bf16 matrix cores
     (2.5 PFLOP/s / 6), the pair_share as fp16-pair products (2.5 PFLOP/s / 3),
     the pair16_share as fp16-pair products on the 16x16x16 instruction
-    (1.25 PFLOP/s / 3), the shortk_share as the short-K kernel's five fp16
+    (1.25 PFLOP/s / 3), the shortk_share as the three-part kernels' five fp16
     products (2.5 PFLOP/s / 5), the rest on the fp32 matrix cores
     (157.3 TFLOP/s)."""
     rest = 1.0 - split_share - pair_share - pair16_share - shortk_share
@@ -242,7 +242,7 @@ def time_ef(device, reps, cpu: bool):
         # contraction bound at the ceilings of the instructions that run: the
         # FLOPs this library's dense kernels launched in one evaluation, by
         # instruction class (pet_gemm_flop_tally: bf16 parts, fp16 pairs, the
-        # short-K kernel's five fp16 products), the rest (rocBLAS's products,
+        # three-part kernels' five fp16 products), the rest (rocBLAS's products,
         # the attention) on the fp32 matrix cores
         _lib.gemm_flop_tally(reset=True)
         o = m.compute(x, True)

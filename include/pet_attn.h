@@ -117,8 +117,8 @@ enum {
                               reference's Recompute::Wide, src/model.cpp:819-860) -- the same results */
   PET_OPT_MODEL_PAIRS = 9, /* the whole evaluation's MLPs: 1 (default) an activation, or its adjoint, that only the
                               next product reads passes to it as block pairs (pet_linear_fused_split_blocks /
-                              pet_linear_fused_blocks) where both products take the pairs-by-pairs kernel; 0 as
-                              fp32 and a split pass */
+                              pet_linear_fused_blocks) where both products run from pairs; 0 as fp32 and a
+                              split pass */
   PET_OPT_COUNT = 10
 };
 

@@ -8,8 +8,9 @@
  * its analytic backward, the readout and energy assembly
  * (src/model.cpp:656-780, src/ops.cpp:406-425) and forces_and_virial
  * (src/forces.cpp:345-386) for a fixed cutoff. Every kernel is this library's
- * (the attention, norms, activations, gathers, folds); the dense layers go to
- * rocBLAS fp32 with atomics off, so results repeat bit for bit.
+ * (the attention, norms, activations, gathers, folds, and the dense layers but
+ * the narrow ones, which go to rocBLAS fp32 with atomics off), so results repeat
+ * bit for bit.
  *
  * Weights come as the checkpoint stores them (include/pet/checkpoint.hpp,
  * src/model.cpp:180-289: torch Linear layout, a SwiGLU w_in as [value | gate]

@@ -307,7 +307,7 @@ def gemm_flop_tally(reset: bool = False) -> dict:
     """FLOPs (2 M N K) of the dense products this library's kernels have
     launched in this process, by instruction class (pet_gemm_flop_tally):
     "fp32" the fp32 fused kernel, "split" bf16 parts (six products), "pair"
-    fp16 pairs (three), "shortk" the short-K kernel (five fp16 products)."""
+    fp16 pairs (three), "shortk" the three-part kernels (five fp16 products)."""
     out = (ctypes.c_double * 4)()
     check(load().pet_gemm_flop_tally(out, int(reset)), "pet_gemm_flop_tally")
     return dict(fp32=out[0], split=out[1], pair=out[2], shortk=out[3])

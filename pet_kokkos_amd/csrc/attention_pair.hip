@@ -43,10 +43,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <map>
-#include <mutex>
 #include <type_traits>
-#include <utility>
 
 #include "../../include/pet_attn.h"
 #include "attn_common.h"
@@ -76,7 +73,8 @@ namespace {
 // kernel, whose products take eight instructions where the pairs take three:
 // 640 atoms of 180 neighbours on MI355X (14 waves, d 256), backward 720 -> 490
 // us (427 with mfma_block), forward 207 -> 173; S 143 (nine waves) 373 -> 280
-// and 114 -> 100.
+// and 114 -> 100. (At head_dim 64 the forward past nine waves, with the fused
+// transform, spills 8 registers, outside its loop over the keys.)
 constexpr int kPairMaxWaves = 16;
 constexpr float kFltMax = 3.40282347e38f;
 constexpr int pair_waves(int NW) { return NW <= 9 ? NW : (NW + 1) & ~1; }
@@ -960,24 +958,6 @@ const void* pair_kernel_nw(int NW, bool x) {
   }
   return nullptr;
 }
-
-// The dynamic LDS limit of kernel k raised, once per device, to the largest
-// size asked.
-int allow_lds_pair(const void* k, size_t bytes) {
-  if (bytes <= 65536) return PET_ATTN_OK;
-  static std::map<std::pair<int, const void*>, size_t> raised;
-  static std::mutex mu;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return PET_ATTN_ELAUNCH;
-  std::lock_guard<std::mutex> lock(mu);
-  size_t& have = raised[{dev, k}];
-  if (have < bytes) {
-    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess)
-      return PET_ATTN_ELAUNCH;
-    have = bytes;
-  }
-  return PET_ATTN_OK;
-}
 }  // namespace
 
 int pair_bwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* qkv, int64_t ldq, const int* off,
@@ -994,7 +974,7 @@ int pair_bwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
   const void* k = qpairs ? (HD == 64 ? pair_kernel_nw<64, true>(NW, x) : pair_kernel_nw<32, true>(NW, x))
                          : (HD == 64 ? pair_kernel_nw<64>(NW, x) : pair_kernel_nw<32>(NW, x));
   if (!k) return PET_ATTN_ESLOTS;
-  if (const int e = allow_lds_pair(k, bytes)) return e;
+  if (const int e = raise_lds(k, bytes)) return e;
   const PairBwdArgs a{qkv,  ldq,    off,    sh.n_atoms, n0,  eb,   sh.slots, sh.heads,
                       sh.scale, dmerged, ldg, merged, ldm, ml, cf_seq, ldc, qkv_adj, lda, cfh, xf,
                       static_cast<u4*>(qpairs), prows};
@@ -1046,7 +1026,7 @@ int pair_fwd(const pet_attn_shape& sh, int n0, int n1, int64_t eb, const float* 
     by_waves(std::integral_constant<int, 64>{});
   else
     by_waves(std::integral_constant<int, 32>{});
-  if (const int e = allow_lds_pair(reinterpret_cast<const void*>(k), bytes)) return e;
+  if (const int e = raise_lds(reinterpret_cast<const void*>(k), bytes)) return e;
   hipLaunchKernelGGL(k, dim3(unsigned(items)), dim3(64 * NW), bytes, st, qkv, ldq, off, sh.n_atoms, n0, eb, sh.slots,
                      sh.heads, sh.scale, cf_seq, ldc, merged, ldm, ml, xf);
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;

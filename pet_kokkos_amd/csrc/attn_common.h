@@ -10,6 +10,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <map>
+#include <mutex>
+#include <utility>
+
+#include "../../include/pet_attn.h"
 
 namespace pet_attn {
 
@@ -169,5 +174,23 @@ __device__ __forceinline__ void store_slice(float* dst, const f4* acc, float f) 
                     tile_elem<DT>(acc, e + 3) * f);
 }
 
+
+// The dynamic LDS limit of kernel k (64 KB by default) raised, once per kernel
+// and device, to the largest size asked.
+inline int raise_lds(const void* k, size_t bytes) {
+  if (bytes <= 65536) return PET_ATTN_OK;
+  static std::map<std::pair<int, const void*>, size_t> raised;
+  static std::mutex mu;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return PET_ATTN_ELAUNCH;
+  std::lock_guard<std::mutex> lock(mu);
+  size_t& have = raised[{dev, k}];
+  if (have < bytes) {
+    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess)
+      return PET_ATTN_ELAUNCH;
+    have = bytes;
+  }
+  return PET_ATTN_OK;
+}
 
 }  // namespace pet_attn

@@ -40,8 +40,6 @@ using pet_split::mfma6;
 using pet_split::pack_hi;
 using pet_split::split3;
 using pet_split::split8;
-using pet_split::mfma3;
-using pet_split::mfma_h;
 using pet_split::pair2;
 using pet_split::pair_scale;
 
@@ -880,8 +878,8 @@ int pet_gemm_nt_pp(int M, int N, int K, const void* Ap, const void* Bs, float* C
 }
 
 // Block pairs out (as pet_gemm_nt_split_pairs) from A already as pair rows
-// (pet_gemm_pair_rows' layout, K of the pair form): the pairs-by-pairs kernel
-// alone, every row at once.
+// (pet_gemm_pair_rows' layout, K of the pair form): gemm_rows_kernel from
+// pairs alone, every row at once.
 int pet_gemm_nt_pp_to_blocks(int M, int N, int K, const void* Ap, const void* Bs, void* pout, const float* bias,
                              const float* cin, int64_t ldcin, float beta, float* pre, int64_t ldpre, int act,
                              hipStream_t st, int* kb) {
@@ -898,7 +896,7 @@ int pet_gemm_nt_pp_to_blocks(int M, int N, int K, const void* Ap, const void* Bs
   return pet_gemm_nt_pp(M, N, K, Ap, Bs, nullptr, 0, e, st);
 }
 
-constexpr int kMaxBlocks = 32;
+constexpr int kMaxBlocks = 32;  // (the interface's limit, of its callers' too; the kernel takes any number)
 
 // C = epi(A B^T) with A as block pairs (pet_gemm_nt_split_pairs' pout: M
 // rows of pairs, then the inverse scales [K / kb][M]) and B's pair rows; kb 32,

@@ -22,8 +22,8 @@
 //     so far of the row's first step in [2^11, 2^12), and a later value past
 //     2^15 lowers it (rare: eight times the first 32 values' largest; the
 //     accumulators are then rescaled by the exact power of two). A value keeps
-//     22 significand bits down to 2^-18 of the row's largest, as under the
-//     row's own scale down to 2^-21.
+//     22 significand bits down to 2^-14 of the row's largest (under the row's own
+//     scale, kExact, to 2^-17), and below an error of at most 2^-36 of it (2^-39).
 //   kExact: the row's largest |x| is found first, in a pass over the wave's rows
 //     (whose second reading comes from cache): the bits of the pair rows
 //     (pair_act_kernel) read in form kPairs.
@@ -31,15 +31,14 @@
 //     sum, made from zero at its block's own scale, is brought to the row's
 //     smallest scale in fp32 as it is added, so that a block far below the row's
 //     largest keeps all of its bits.
-// A row's results depend on that row alone, and repeat bit for bit.
+// In one kernel a row's results depend on that row alone, and repeat bit for bit.
+// The tile kernel's shapes and the strip share one order of sums; the kernel that
+// splits K over its waves (three parts, K from 256, few rows) has its own.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
-#include <map>
-#include <mutex>
 #include <type_traits>
-#include <utility>
 
 #include "../../include/pet_model.h"
 #include "attn_common.h"
@@ -840,8 +839,7 @@ gemm_strip_kernel(int M, int N, const float* A, int64_t lda, const u4* B, float*
   for (int p = 0; p < 3; ++p) sb[p] = swizzle<3>(3 * g + p, c);
   const float* inv_b = reinterpret_cast<const float*>(B + int64_t(N) * KG * 3);
   for (; blk < nb; blk += NW * S) {
-    // the block's loads done (issued before the last block's epilogue, whose
-    // stores, at least NST of them, may still be on their way)
+    // (the block's loads are done: waited for after the last block's epilogue)
     u4 ah[KB], al[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) ah[k] = slice[(16 * k + c) * 8 + s0], al[k] = slice[(16 * k + c) * 8 + s1];
@@ -953,34 +951,24 @@ template <int TM, int NW, int OUT>
 RowsShape ksplit_shape() {
   return {gemm_ksplit_kernel<TM, 4, NW, OUT>, 16 * TM, 64, 64 * NW, size_t(NW) * (16 * TM * 8 + 64 * 12) * 16};
 }
-// A kernel's dynamic LDS above the 64 KB default, once a kernel and device.
-int allow_lds_rows(const void* k, size_t bytes) {
-  if (bytes <= 65536) return PET_ATTN_OK;
-  static std::map<std::pair<int, const void*>, size_t> raised;
-  static std::mutex mu;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return PET_ATTN_ELAUNCH;
-  std::lock_guard<std::mutex> lock(mu);
-  size_t& have = raised[{dev, k}];
-  if (have < bytes) {
-    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)) != hipSuccess) return PET_ATTN_ELAUNCH;
-    have = bytes;
-  }
-  return PET_ATTN_OK;
-}
-// The shapes: 1 256 x 256 of 64 x 128 a wave (two parts), 2 128 x 128 of 64 x
-// 64, 3 64 x 128 of 32 x 64, 4 64 x 64 of 32 x 32, 5 64 x 32 of 16 x 32; block
+// The shapes: 1 256 x 256 of 64 x 128 a wave, 2 128 x 128 of 64 x 64 (both two
+// parts), 3 64 x 128 of 32 x 64, 4 64 x 64 and 5 32 x 64 of 16 x 64; 7, 8 and 9 64,
+// 32 and 16 x 64 with the steps split over four waves (three parts); block
 // pairs out (a wave 128 columns, a block of the output): 1, and 6 128 x 128 of
-// 32 x 128.
+// 32 x 128. Shape 1 needs more than its 256 registers: with block pairs out it
+// spills 70 (124 bytes a lane), in the epilogue, from fp32 rows 3; the 128-column
+// strip spills 16.
 template <int P, int AS, int OUT>
 RowsShape rows_pick(int cfg) {
   if constexpr (OUT == kBlocks) {
     if (cfg == 1) return rows_shape<4, 8, 4, 2, P, AS, OUT>();
     return rows_shape<2, 8, 4, 1, P, AS, OUT>();
   } else {
-    if constexpr (P == 2 && OUT == kVec)
-      if (cfg == 1) return rows_shape<4, 8, 4, 2, P, AS, OUT>();
-    if (cfg <= 2) return rows_shape<4, 4, 2, 2, P, AS, OUT>();
+    if constexpr (P == 2) {
+      if constexpr (OUT == kVec)
+        if (cfg == 1) return rows_shape<4, 8, 4, 2, P, AS, OUT>();
+      if (cfg <= 2) return rows_shape<4, 4, 2, 2, P, AS, OUT>();
+    }
     if (cfg == 3) return rows_shape<2, 4, 2, 2, P, AS, OUT>();
     if (cfg == 4) return rows_shape<1, 4, 4, 1, P, AS, OUT>();
     if constexpr (AS == kOnline && P == 3) {
@@ -997,7 +985,8 @@ RowsShape rows_pick(int cfg) {
 // from K = 256: 2; pet_gemm_pair_weights: 3); as: how A comes (kOnline,
 // kExact: fp32 rows, 16-byte aligned; kPairs: pair rows or blocks of kb
 // columns). K a multiple of 32; e.pout: block pairs in place of C (N a multiple
-// of 128, A as pairs, every operand 16-byte aligned). cfg: the shape (0: chosen here).
+// of 128, A as pairs, every operand 16-byte aligned). cfg: the shape (0, with two
+// parts: chosen here).
 int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, int kb, const void* Bp, int P, float* C,
                      int64_t ldc, const Epi& e, hipStream_t st, int cfg) {
   if (M < 0 || N < 0 || K < 32 || K % 32 || (as == kPairs && (kb < 32 || kb % 32 || K % kb))) return PET_ATTN_EINVAL;
@@ -1008,11 +997,14 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
   const bool vec = N % 4 == 0;
   auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(64, 32) >= (int64_t(1) << 31)) return PET_ATTN_EINDEX;
+  if (P == 3 && (cfg < 3 || cfg == 6)) return PET_ATTN_EINVAL;
   if (!cfg) {
     // 256 x 256 tiles (one workgroup a CU) where their last round of 256 leaves
     // at most a sixth of the CUs idle over all rounds: full, they are 1.13 to 1.17 times
     // faster than 128 x 128 (62291 x 512 x 1024 from pairs: 176 against 204 us, 488
-    // tiles; 26670 x 1024 x 512 with SwiGLU: 102 against 94, 420 tiles). An
+    // tiles, 95% of their rounds full; at 82%, 26670 x 1024 x 512 with SwiGLU, 102
+    // against 94; at 83%, 217834 x 256 x 768, 281 against 291: the line could lie a
+    // hundredth lower). An
     // activation's backward into block pairs is bound by its operand: 128 x 128
     // there (62291 x 1024 x 512, SwiGLU: 324 against 382). A width that is no
     // multiple of 4 keeps to 128 x 128: with its last columns one by one the
@@ -1022,7 +1014,7 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
     if (e.pout)
       cfg = c1 && N % 256 == 0 && e.act <= 2 ? 1 : 6;
     else
-      cfg = P == 2 && c1 ? 1 : N > 64 && tiles(128, 128) >= 512 ? 2 : N > 64 && tiles(64, 128) > 256 ? 3 : tiles(64, 64) >= 256 ? 4 : 5;
+      cfg = c1 ? 1 : N > 64 && tiles(128, 128) >= 512 ? 2 : N > 64 && tiles(64, 128) > 256 ? 3 : tiles(64, 64) >= 256 ? 4 : 5;
   }
   RowsShape s;
   using std::integral_constant;
@@ -1038,7 +1030,7 @@ int pet_gemm_nt_rows(int M, int N, int K, const void* A, int64_t lda, int as, in
   else if (P == 2 && as == kExact) pick(integral_constant<int, 2>{}, integral_constant<int, kExact>{});
   else if (P == 2 && as == kPairs) pick(integral_constant<int, 2>{}, integral_constant<int, kPairs>{});
   if (!s.k) return PET_ATTN_EINVAL;
-  if (const int rc = allow_lds_rows(reinterpret_cast<const void*>(s.k), s.lds)) return rc;
+  if (const int rc = pet_attn::raise_lds(reinterpret_cast<const void*>(s.k), s.lds)) return rc;
   // windows of row blocks where the weights pass an L2's share
   const int win = int64_t(N) * K * 2 * P > (2 << 20) ? 4 : 1;
   hipLaunchKernelGGL(s.k, dim3(unsigned(tiles(s.bm, s.bn))), dim3(s.threads), s.lds, st, M, N, K, A, lda,
@@ -1088,7 +1080,7 @@ int pet_gemm_nt_strip(int M, int N, int K, const float* A, int64_t lda, const vo
   if (BN == 128) by_k(std::integral_constant<int, 8>{});
   else by_k(std::integral_constant<int, 4>{});
   const size_t bytes = size_t(KB) * (BN * 12 + 8 * 128) * 16;
-  if (const int rc = allow_lds_rows(reinterpret_cast<const void*>(k), bytes)) return rc;
+  if (const int rc = pet_attn::raise_lds(reinterpret_cast<const void*>(k), bytes)) return rc;
   hipLaunchKernelGGL(k, dim3(unsigned(8 * NT * S)), dim3(512), bytes, st, M, N, A, lda, static_cast<const u4*>(Bp), C, ldc, e, S);
   tally(3, M, N, K);
   return hipGetLastError() == hipSuccess ? PET_ATTN_OK : PET_ATTN_ELAUNCH;

@@ -8,7 +8,8 @@
 // (attention.hip), the norms (rows.hip), the edge term and folds (forces.hip)
 // and, here, the gathers, compress.0's folded form, SiLU / SwiGLU and their
 // backwards, the residual sums, the combination's concat and the readout. The
-// dense layers go to rocBLAS fp32 (ops.hip's gemm_nt / gemm_nn, atomics off).
+// dense layers go to this library's kernels (gemm_rows.hip, gemm.hip), a few to
+// rocBLAS fp32 (ops.hip's gemm_nt / gemm_nn, atomics off): split_for.
 // The elementwise passes are HBM-bound: grid-stride loops over contiguous
 // row-major buffers, one read and one write per value, residual sums fused
 // into the pass that produces their operands.
@@ -612,7 +613,7 @@ struct pet_model {
 namespace {
 
 // Which forward dense layers take this library's fused GEMM (gemm.hip) instead
-// of rocBLAS: 0 none (the default), 1 all, 2 those with at most 4096 rows.
+// of the kernels that split_for chooses: modes 1 all, 2 those with at most 4096 rows.
 // Measured on MI355X (C2 / C2-residual / C5 energy+forces, ms): 3.45 / 2.67 /
 // 281 with rocBLAS, 3.50 / 2.68 / 281 with mode 2, 3.96 / 3.00 / 311 with mode
 // 1: its main loop reaches 72% of the fp32 matrix peak at K = 1024 where
@@ -633,10 +634,9 @@ bool own_gemm(const pet_model& md, int M, int K) {
 // for K at most 128, the split-product kernel above -- so that no result depends
 // on how many rows come with it; 3 the split-product kernel for every product;
 // 0 rocBLAS only. The narrow products (N < 64: the readout's) stay on rocBLAS in
-// mode 6: the matrix instruction truncates each product toward zero below the
-// result's last place, and with a fixed weight vector and mostly positive
-// inputs those truncations share a sign on every atom and add up over a
-// structure (C2-residual 5.7e-7 with them on it).
+// mode 6, where nothing speaks for either: on the three-part kernels the evaluations
+// take the same time (within 0.4%, three workloads on MI355X), and from float64 their
+// energies are 3 to 6% further off and their forces 8 to 15% nearer.
 // The kernel a product takes (null: rocBLAS): the copy of W it reads and
 // whether that is the three-part one.
 struct Sel {

@@ -102,12 +102,12 @@ int split_dense(float* out, int64_t ldo, const float* A, int64_t lda, const floa
   if (int e = pet_gemm_pair_weights(W, N, K, ldw, W_is_bt, split, st)) return e;
   return pet_gemm_nt_parts(M, N, K, A, lda, split, out, ldo, nullptr, bias, cin, ldo, beta, nullptr, 0, 0, st);
 }
-// Bytes of the layer level's room for split weights: W_in (folded) or W_in^T
-// [3D x D], W_out or W_out^T [D x D].
+// Bytes of the layer level's room for a split weight, one at a time: the largest,
+// W_in (folded) or W_in^T [3D x D], in three parts.
 inline size_t align256s(size_t n) { return (n + 255) & ~size_t(255); }
 size_t layer_split_bytes(int D) {
   const size_t d = size_t(D);
-  return 2 * align256s(6 * 3 * d * d) + 2 * align256s(6 * d * d);
+  return align256s(6 * 3 * d * d + 4 * 3 * d);
 }
 
 // out[r][j] = b[j] (or 0 without a bias): the bias the GEMM then accumulates onto.
@@ -457,7 +457,7 @@ int pet_attention_layer(const pet_attn_shape* sh, float* out, int64_t ldo, const
   float* normed = reinterpret_cast<float*>(ws);
   float* qkv = reinterpret_cast<float*>(ws + a0);
   // a weight's split copy, made before its product in the place of the last one's
-  // (6 N K + 4 N bytes at most of layer_split_bytes), past the backward's workspace
+  // (layer_split_bytes), past the backward's workspace
   char* sp = ws + a0 + a1 + a2 + align256(sizeof(float) * 3 * size_t(D) * D) + pet_attention_bwd_workspace(sh);
   if (!norm_b) {  // RMSNorm: the fused projection, norm and bias applied by the attention
     float *inv = reinterpret_cast<float*>(ws + a0 + a1), *wf = reinterpret_cast<float*>(ws + a0 + a1 + a2);

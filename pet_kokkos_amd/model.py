@@ -276,8 +276,8 @@ def ef_gemms(h: Hypers, n_atoms: int, n_edges: int) -> list:
 
 # The model's dense products with M N K >= 2^32 run on the split-product kernel
 # by default (fp32 accuracy on the 16-bit matrix cores: from K = 256 as fp16
-# pairs, three products; below as three bf16 parts, six products); the rest on
-# rocBLAS fp32.
+# pairs, three products; below as three bf16 parts, six products); the rest with
+# N >= 64 on the three-part kernels, the narrow ones on rocBLAS fp32.
 SPLIT_THRESHOLD = 2.0 ** 32
 PAIR_MIN_K = 256
 

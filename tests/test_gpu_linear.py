@@ -29,8 +29,8 @@ def linear_fused(A, W, C, row_scale=None, bias=None, cin=None, beta=0.0, pre=Non
 
 
 # the last two are large enough for the split form's 128 x 128 and 128 x 64 tiles
-# (1001, 38, 96): a width not a multiple of 4 (the short-K kernel's per-element
-# epilogue) and 12 k groups a row (its rows padded to 16 lanes); (3, 130, 64),
+# (1001, 38, 96): a width not a multiple of 4 (the epilogues' last columns one
+# by one) and 12 k groups a row; (3, 130, 64),
 # (5, 130, 128): fewer rows than one block, most XCDs' row ranges empty
 SHAPES = [(1, 16, 16), (37, 40, 32), (300, 128, 128), (2049, 96, 256), (5000, 384, 128), (1000, 1024, 512),
           (129, 64, 1024), (16385, 1024, 64), (131071, 96, 64), (1001, 38, 96), (3, 130, 64), (5, 130, 128)]
@@ -414,7 +414,7 @@ def test_smallk_rows_independent_of_M(K, device):
 
 
 def smallk_parts(W):
-    """The short-K weights' parts [N, K/8, 3, 8] (hi, mid, lo) and inverse scales [N], fp64."""
+    """The three-part weights' parts [N, K/8, 3, 8] (hi, mid, lo) and inverse scales [N], fp64."""
     N, K = W.shape
     raw = W.data.cpu().numpy().view(np.uint8)
     parts = raw[: N * K * 6].view(np.float16).reshape(N, K // 8, 3, 8).astype(np.float64)
@@ -423,7 +423,7 @@ def smallk_parts(W):
 
 
 def W_ref(W, device):
-    """The fp64 matrix of part weights over each row's scale: the short-K
+    """The fp64 matrix of part weights over each row's scale: the three-part
     weights' hi + mid + lo, or the pair form's hi + lo (SplitWeights from
     K = 256)."""
     N, K = W.shape
@@ -442,7 +442,7 @@ def test_smallk_weights_exact(device):
     [2^14, 2^15)), per element hi = w s to the nearest fp16, mid = the rest to
     the nearest fp16, lo = what is left: hi + mid + lo = w s exactly wherever
     |w s| >= 2^-1 (lo then holds at most 2 bits at an exponent fp16 reaches),
-    within half an fp16 subnormal step below. So the weights the short-K
+    within half an fp16 subnormal step below. So the weights the three-part
     kernel multiplies are W itself: a pair form (22 bits) would be a fixed
     perturbation of the model, the same error in every row's product."""
     N, K = 40, 128
@@ -606,7 +606,7 @@ def test_norm_pair_rows_same_bits(K, device):
 
 def test_flop_tally(device):
     """pet_gemm_flop_tally: each launch adds 2 M N K to its instruction class
-    (the short-K kernel's, the fp32 fused kernel's), and reset zeroes them."""
+    (the three-part kernels', the fp32 fused kernel's), and reset zeroes them."""
     _lib.gemm_flop_tally(reset=True)
     M, N, K = 1000, 96, 64
     g = torch.Generator(device=device).manual_seed(70)
@@ -646,7 +646,7 @@ def test_three_part_kernels_long_k(M, N, K, device):
 
 
 def three_part_kernels(M, N, K, device, alone):
-    """The short-K layer's kernels over their dispatch, with rows over 40
+    """The three-part kernels over their dispatch, with rows over 40
     octaves, rows that outgrow their first 32 values by up to 2^20 (the running
     scale), zero rows, and every epilogue. An element's error is bounded by
     2^-20 of sum |a| |w|: the rows' pairs hold 24 bits less a half (2^-24), each

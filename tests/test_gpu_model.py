@@ -27,9 +27,9 @@ error an fp32 restatement of the reference makes on the same structure where
 fp32 itself cannot meet it. On C2's water-648 the tests also assert fixed bars
 that the float32 oracle meets as well: energy 5e-7 relative, forces 5e-5
 eV/A. Measured on
-MI355X, C2 water-648: energy 3.0e-7 relative (float32 oracle 3.3e-7), forces
-2.0e-5 eV/A (float32 oracle 2.6e-5); residual family 3.8e-7 (4.2e-7) and
-1.2e-5 (1.7e-5) eV/A; against the float32 oracle, energy 3.4e-8 and 4.1e-8
+MI355X, C2 water-648: energy 2.1e-7 relative (float32 oracle 3.3e-7), forces
+1.4e-5 eV/A (float32 oracle 2.6e-5); residual family 4.5e-7 (4.2e-7) and
+6.1e-6 (1.7e-5) eV/A; against the float32 oracle, energy 1.2e-7 and 3.3e-8
 relative. Runs repeat bit for bit.
 """
 from __future__ import annotations
@@ -147,7 +147,7 @@ def test_model_on_the_fused_dense_layer(name, mode, device):
     # on the library's fused GEMM (pet_linear_fused's kernel) instead of
     # rocBLAS; 3: every dense layer with K a multiple of 32 on its
     # split-product form (pet_linear_fused_split's kernel), backward included;
-    # 6: the short-K kernel for the K <= 128 layers with a bias or activation
+    # 6, the default: the three-part kernels but for the large products
     from pet_kokkos_amd import _lib
     h = weights.MODELS[name]
     w = weights.random_weights(h, 15)
@@ -213,11 +213,10 @@ def fixed_bars(name, got, ref, e_bar=5e-7, f_bar=5e-5):
     not this library's): energy 5e-7 relative, forces 5e-5 eV/A against the
     float64 oracle. Then the north star's literal comparison, the GPU against
     an fp32 pipeline (the float32 oracle standing for the reference's):
-    energy 1e-7 relative and forces 1e-5 eV/A where the two fp32 evaluations'
-    own distances to float64 leave room for it; where they do not, the GPU's
-    distance to the float32 oracle is held to the sum of the two distances
-    (the float32 oracle's own miss plus this library's, each within the bars
-    above), and the numbers are printed."""
+    energy 1e-7 relative and forces 1e-5 eV/A where fp32 can meet it, that is
+    where the float32 oracle's own distance to float64 is not more; else twice
+    that distance, which an evaluation no further from float64 than the float32
+    oracle cannot pass. The numbers are printed."""
     e64, f64 = ref["energy"], ref["forces"]
     e_gpu, f_gpu = got["energy"].cpu().numpy(), got["forces"].cpu().numpy()
     e32, f32 = ref["fp32"]["energy"], ref["fp32"]["forces"]
@@ -228,11 +227,11 @@ def fixed_bars(name, got, ref, e_bar=5e-7, f_bar=5e-5):
         assert de <= e_bar and df <= f_bar, name_
     de = np.max(np.abs(e_gpu - e32) / np.abs(e32))
     df = np.abs(f_gpu - f32).max()
-    room_e = np.max(np.abs(e_gpu - e64) / np.abs(e64)) + np.max(np.abs(e32 - e64) / np.abs(e64))
-    room_f = np.abs(f_gpu - f64).max() + np.abs(f32 - f64).max()
+    miss_e = np.max(np.abs(e32 - e64) / np.abs(e64))
+    miss_f = np.abs(f32 - f64).max()
     print(f"[model] {name}: gpu against the float32 oracle (the north star's literal bar 1e-7, 1e-5): "
           f"energy {de:.2e} relative, forces {df:.2e} eV/A", flush=True)
-    assert de <= max(1e-7, room_e * (1 + 1e-6)) and df <= max(1e-5, room_f * (1 + 1e-6))
+    assert de <= max(1e-7, 2 * miss_e) and df <= max(1e-5, 2 * miss_f)
 
 
 def test_calculator(device):
