@@ -250,7 +250,7 @@ __device__ __forceinline__ void put_cols(float* p, const float (&x)[n], int left
 // and the columns' inv_b (a row past 2^64 apart from that factor of its scale,
 // which follows inv_b: sums of 2^30 and more times a scale up to 2^116 can pass the
 // range of a float where the result does not; FAR: three-part weights, whose
-// products ran in fp32, and block pairs out, whose kernel spills 70 registers
+// products ran in fp32, and block pairs out, whose kernel spills 69 registers
 // with it and 101 without), then epi_elem's arithmetic in its order. A lane holds
 // sixteen consecutive columns of its row c; a 4 x 4 transpose of those 16-byte
 // chunks over each quad of lanes makes an instruction's quad cover 64 bytes of
@@ -504,12 +504,20 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   for (int s = 0; s < ST - 1; ++s) issue(s, s);
 
   f4 ts[NG > 1 ? 2 : 1][TM][TG];  // a group's step
-  auto add_group = [&](auto set, int bg) {
+  // kExact: the running sum turned with the steps' sign (turn: t - acc, the sign of
+  // the last step at the end) in a K loop of its own: with the sign a multiplier,
+  // as in the other forms, the 256 x 256 tiles spill in the loop (62291 x 1024 x 512
+  // 290 us against 259)
+  auto add_group = [&](auto set, int bg, auto turn) {
     constexpr int X = decltype(set)::value;
 #pragma unroll
     for (int j = 0; j < TG; ++j)
 #pragma unroll
-      for (int a = 0; a < TM; ++a) add_step(acc[a][TG * bg + j], ts[X][a][j], AS == kPairs ? fac[a] : sg);
+      for (int a = 0; a < TM; ++a) {
+        f4& s = acc[a][TG * bg + j];
+        if constexpr (AS == kExact) s = turn ? ts[X][a][j] - s : ts[X][a][j] + s;
+        else add_step(s, ts[X][a][j], AS == kPairs ? fac[a] : sg);
+      }
   };
   using last_ = std::integral_constant<int, (NG > 1 ? 1 : 0)>;  // the last group's set
   int stage = 0;          // step s's
@@ -519,113 +527,125 @@ gemm_rows_kernel(int M, int N, int K, const void* A, int64_t lda, const u4* B, f
   int sb[P];
 #pragma unroll
   for (int p = 0; p < P; ++p) sb[p] = swizzle<P>(g * P + p, c);
-  for (int s = 0; s < steps; ++s) {
-    // the step's stage in LDS for this wave's loads (those of the stages after
-    // it may still fly), then for every wave's; no wave still reads the stage
-    // of step s - 1, which the next loads fill
-    wait_vm<(ST - 2) * (LA + (NIB % NW == 0 ? LB : LB - 1))>();
-    ring_barrier();
-    issue(s + ST - 1, stage == 0 ? ST - 1 : stage - 1);
-    const u4* at = lds + stage * Sh::STAGE + ar * 8;
-    const u4* bt = lds + stage * Sh::STAGE + BM * 8 + bc * CH;
-    u4 ah[TM], al[TM];
+  auto k_loop = [&](auto turn) {
+    for (int s = 0; s < steps; ++s) {
+      // the step's stage in LDS for this wave's loads (those of the stages after
+      // it may still fly), then for every wave's; no wave still reads the stage
+      // of step s - 1, which the next loads fill
+      wait_vm<(ST - 2) * (LA + (NIB % NW == 0 ? LB : LB - 1))>();
+      ring_barrier();
+      issue(s + ST - 1, stage == 0 ? ST - 1 : stage - 1);
+      const u4* at = lds + stage * Sh::STAGE + ar * 8;
+      const u4* bt = lds + stage * Sh::STAGE + BM * 8 + bc * CH;
+      u4 ah[TM], al[TM];
 #pragma unroll
-    for (int a = 0; a < TM; ++a) {
-      ah[a] = at[(16 * a + c) * 8 + sa0];
-      al[a] = at[(16 * a + c) * 8 + sa1];
-    }
-    // B's operands a group of TG tiles ahead of its products (the scheduling
-    // barriers keep the reads there: left alone, the compiler reads each
-    // group's operands just before its products and waits)
-    u4 wv[2][TG][P];
-    auto read = [&](auto set, int bg) {
-      constexpr int X = decltype(set)::value;
-#pragma unroll
-      for (int j = 0; j < TG; ++j)
-#pragma unroll
-        for (int p = 0; p < P; ++p) wv[X][j][p] = bt[(16 * (TG * bg + j) + c) * CH + sb[p]];
-    };
-    using c0_ = std::integral_constant<int, 0>;
-    using c1_ = std::integral_constant<int, 1>;
-    read(c0_{}, 0);
-    if constexpr (NG > 1) read(c1_{}, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (s) add_group(last_{}, NG - 1);
-    sg = __uint_as_float(0x3f800000u | (s & 1 ? alt : 0u));
-    if constexpr (AS == kPairs) {
-#pragma unroll
-      for (int a = 0; a < TM; ++a) fac[a] = copysignf(fac[a], sg);
-      if (kbs < steps) {
-        if (left == 0) {  // a block begins: its factor, and the next one's scale on its way
-          left = kbs, blk = min(blk + 1, steps / kbs - 1);
-#pragma unroll
-          for (int a = 0; a < TM; ++a) {
-            fac[a] = sg * inext[a] * __uint_as_float((254 - (imax >> (8 * a) & 255)) << 23);
-            inext[a] = inv_a[int64_t(blk) * M + min(m0 + 16 * a + c, M - 1)];
-          }
-        }
-        --left;
+      for (int a = 0; a < TM; ++a) {
+        ah[a] = at[(16 * a + c) * 8 + sa0];
+        al[a] = at[(16 * a + c) * 8 + sa1];
       }
-    } else {
-      if constexpr (AS == kExact) {
-        if (s == 0)
-#pragma unroll
-          for (int a = 0; a < TM; ++a) sa[a] = pet_split::pair_scale(smax[ar + 16 * a + c]);
-      } else {
-        float m[TM];
-        bool over = false;
-#pragma unroll
-        for (int a = 0; a < TM; ++a) {
-          m[a] = amax8(ah[a], al[a]);
-          over |= m[a] > lim[a];
-        }
-        if (__builtin_amdgcn_ballot_w64(over) != 0) {  // a row outgrew its scale
-#pragma unroll
-          for (int a = 0; a < TM; ++a) {
-            const float f = outgrow(m[a], sa[a], lim[a]);
-#pragma unroll
-            for (int b = 0; b < TN; ++b) acc[a][b] *= f;
-          }
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < TM; ++a) split8x(ah[a], al[a], P == 3 ? sg * sa[a] : sa[a]);
-    }
-    // the small products first, TG TM independent sums between two dependent
-    // ones; a group's step is added under the next group's products
-    auto products = [&](auto set, int bg) {
-      constexpr int X = decltype(set)::value;
-#pragma unroll
-      for (int j = 0; j < TG; ++j)
-#pragma unroll
-        for (int a = 0; a < TM; ++a) ts[X][a][j] = f4{0.f, 0.f, 0.f, 0.f};
-      auto prod = [&](int p, const u4* a_) {
+      // B's operands a group of TG tiles ahead of its products (the scheduling
+      // barriers keep the reads there: left alone, the compiler reads each
+      // group's operands just before its products and waits)
+      u4 wv[2][TG][P];
+      auto read = [&](auto set, int bg) {
+        constexpr int X = decltype(set)::value;
 #pragma unroll
         for (int j = 0; j < TG; ++j)
 #pragma unroll
-          for (int a = 0; a < TM; ++a) ts[X][a][j] = mfma_h(wv[X][j][p], a_[a], ts[X][a][j]);
+          for (int p = 0; p < P; ++p) wv[X][j][p] = bt[(16 * (TG * bg + j) + c) * CH + sb[p]];
       };
-      if constexpr (P == 2) {
-        prod(0, al), prod(1, ah), prod(0, ah);
-      } else {
-        prod(1, al), prod(2, ah), prod(0, al), prod(1, ah), prod(0, ah);
-      }
-      if (bg > 0) add_group(std::integral_constant<int, X ^ 1>{}, bg - 1);
-    };
-#pragma unroll
-    for (int bg = 0; bg < NG; bg += 2) {
-      products(c0_{}, bg);
-      if (bg + 2 < NG) read(c0_{}, bg + 2);
+      using c0_ = std::integral_constant<int, 0>;
+      using c1_ = std::integral_constant<int, 1>;
+      read(c0_{}, 0);
+      if constexpr (NG > 1) read(c1_{}, 1);
       __builtin_amdgcn_sched_barrier(0);
-      if (bg + 1 < NG) {
-        products(c1_{}, bg + 1);
-        if (bg + 3 < NG) read(c1_{}, bg + 3);
-        __builtin_amdgcn_sched_barrier(0);
+      if (s) add_group(last_{}, NG - 1, turn);
+      if constexpr (AS != kExact) sg = __uint_as_float(0x3f800000u | (s & 1 ? alt : 0u));
+      if constexpr (AS == kPairs) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a) fac[a] = copysignf(fac[a], sg);
+        if (kbs < steps) {
+          if (left == 0) {  // a block begins: its factor, and the next one's scale on its way
+            left = kbs, blk = min(blk + 1, steps / kbs - 1);
+#pragma unroll
+            for (int a = 0; a < TM; ++a) {
+              fac[a] = sg * inext[a] * __uint_as_float((254 - (imax >> (8 * a) & 255)) << 23);
+              inext[a] = inv_a[int64_t(blk) * M + min(m0 + 16 * a + c, M - 1)];
+            }
+          }
+          --left;
+        }
+      } else {
+        if constexpr (AS == kExact) {
+          if (s == 0)
+#pragma unroll
+            for (int a = 0; a < TM; ++a) sa[a] = pet_split::pair_scale(smax[ar + 16 * a + c]);
+        } else {
+          float m[TM];
+          bool over = false;
+#pragma unroll
+          for (int a = 0; a < TM; ++a) {
+            m[a] = amax8(ah[a], al[a]);
+            over |= m[a] > lim[a];
+          }
+          if (__builtin_amdgcn_ballot_w64(over) != 0) {  // a row outgrew its scale
+#pragma unroll
+            for (int a = 0; a < TM; ++a) {
+              const float f = outgrow(m[a], sa[a], lim[a]);
+#pragma unroll
+              for (int b = 0; b < TN; ++b) acc[a][b] *= f;
+            }
+          }
+        }
+#pragma unroll
+        for (int a = 0; a < TM; ++a) split8x(ah[a], al[a], P == 3 ? sg * sa[a] : sa[a]);
       }
+      // the small products first, TG TM independent sums between two dependent
+      // ones; a group's step is added under the next group's products
+      auto products = [&](auto set, int bg) {
+        constexpr int X = decltype(set)::value;
+#pragma unroll
+        for (int j = 0; j < TG; ++j)
+#pragma unroll
+          for (int a = 0; a < TM; ++a) ts[X][a][j] = f4{0.f, 0.f, 0.f, 0.f};
+        auto prod = [&](int p, const u4* a_) {
+#pragma unroll
+          for (int j = 0; j < TG; ++j)
+#pragma unroll
+            for (int a = 0; a < TM; ++a) ts[X][a][j] = mfma_h(wv[X][j][p], a_[a], ts[X][a][j]);
+        };
+        if constexpr (P == 2) {
+          prod(0, al), prod(1, ah), prod(0, ah);
+        } else {
+          prod(1, al), prod(2, ah), prod(0, al), prod(1, ah), prod(0, ah);
+        }
+        if (bg > 0) add_group(std::integral_constant<int, X ^ 1>{}, bg - 1, turn);
+      };
+#pragma unroll
+      for (int bg = 0; bg < NG; bg += 2) {
+        products(c0_{}, bg);
+        if (bg + 2 < NG) read(c0_{}, bg + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (bg + 1 < NG) {
+          products(c1_{}, bg + 1);
+          if (bg + 3 < NG) read(c1_{}, bg + 3);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      stage = stage + 1 == ST ? 0 : stage + 1;
     }
-    stage = stage + 1 == ST ? 0 : stage + 1;
+    add_group(last_{}, NG - 1, turn);
+  };
+  if (AS == kExact && alt) {
+    k_loop(std::true_type{});
+    if (!(steps & 1))  // the last step's sign (a zero stays +0)
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f} - acc[a][b];
+  } else {
+    k_loop(std::false_type{});
   }
-  add_group(last_{}, NG - 1);
   wait_vm<0>();  // no load into LDS outlives the loop
   if constexpr (AS == kOnline)
 #pragma unroll
@@ -955,9 +975,8 @@ RowsShape ksplit_shape() {
 // parts), 3 64 x 128 of 32 x 64, 4 64 x 64 and 5 32 x 64 of 16 x 64; 7, 8 and 9 64,
 // 32 and 16 x 64 with the steps split over four waves (three parts); block
 // pairs out (a wave 128 columns, a block of the output): 1, and 6 128 x 128 of
-// 32 x 128. Shape 1 needs more than its 256 registers: with block pairs out it
-// spills 70 (124 bytes a lane), in the epilogue, from fp32 rows 3; the 128-column
-// strip spills 16.
+// 32 x 128. With block pairs out shape 1 needs more than its 256 registers: it spills
+// 69 (120 bytes a lane) in the epilogue; the 128-column strip spills 16.
 template <int P, int AS, int OUT>
 RowsShape rows_pick(int cfg) {
   if constexpr (OUT == kBlocks) {
