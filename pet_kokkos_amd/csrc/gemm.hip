@@ -521,7 +521,7 @@ __global__ void __launch_bounds__(256) pair_rows_kernel(const float* __restrict_
     float carry = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float sj = alt && (j & 4) ? -s : s;
+      const float sj = P == 2 && alt && (j & 4) ? -s : s;
       const float x = at(8 * j + 2 * e) * sj, y = at(8 * j + 2 * e + 1) * sj;
       unsigned h, md, lw;
       if constexpr (P == 2) {
