@@ -20,6 +20,7 @@ device memory and the stream.
 from __future__ import annotations
 
 import dataclasses
+import math
 
 import torch
 
@@ -95,8 +96,14 @@ def _stream() -> int:
 
 def shape(N: int, T: int, S: int, heads: int, head_dim: int, temperature: float = 1.0,
           dead: bool = False) -> _lib.Shape:
-    lib = _lib.load()
-    return _lib.Shape(N, T, S, heads, head_dim, int(dead), lib.pet_attn_scale(head_dim, temperature))
+    # pet_attn_scale's own arithmetic, rounded to float by the struct: a call of the
+    # library less in a forward and in a backward, whose host side is what a small
+    # cell's attention waits for
+    if type(head_dim) is int and type(temperature) is float and head_dim > 0 and temperature > 0.0:
+        scale = 1.0 / (math.sqrt(head_dim) * temperature)
+    else:
+        scale = _lib.load().pet_attn_scale(head_dim, temperature)
+    return _lib.Shape(N, T, S, heads, head_dim, int(dead), scale)
 
 
 def attn_fwd(qkv: torch.Tensor, off: torch.Tensor, cf_seq: torch.Tensor, heads: int, head_dim: int,

@@ -123,3 +123,14 @@ def test_model_create_rejects_before_the_device():
     assert "missing" in _lib.strerror(20)
     lib = _lib.load()
     assert lib.pet_model_compute(None, None, 1, None, None, None, None, None, None) == _lib.EINVAL
+
+
+@pytest.mark.parametrize("temperature", [1.0, 0.5, 1e-3, 3.7, 1e30, 1e-310, float("inf"), 0.0, -1.0, float("nan"), 2])
+def test_shape_scale_is_the_library_s(temperature):
+    """attention.shape makes the scale in Python for a positive float temperature:
+    the same float as pet_attn_scale's, whatever the arguments."""
+    from pet_kokkos_amd import attention
+    lib = _lib.load()
+    for hd in (1, 16, 31, 32, 64, 127, 128):
+        got, want = attention.shape(4, 8, 3, 2, hd, temperature).scale, lib.pet_attn_scale(hd, temperature)
+        assert np.float32(got).tobytes() == np.float32(want).tobytes()
